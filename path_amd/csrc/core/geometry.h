@@ -113,6 +113,20 @@ PT_INLINE bool hit_before(T t, uint32_t idx, T best_t, uint32_t best_idx) {
   return t < best_t || (t == best_t && idx < best_idx);
 }
 
+// False for rays that can hit nothing: those with a NaN component or an
+// infinite direction. Either makes t = f * z of intersect_triangle zero or NaN
+// (a = dot(e1, h) is infinite or NaN for such a direction, where 0 * inf is NaN
+// and no term drops out, and z is NaN for such an origin), which is no t above
+// 1e-5. A tree traversal has to know, since the minima and maxima of the box
+// test skip NaN and every box counts as entered: one such ray (a path in 10^7
+// on the 82k-triangle scene's glass) walked the whole tree alone for 80 ms, of
+// an image that takes 18.
+template <class T> PT_INLINE bool ray_can_hit(const Ray<T> &r) {
+  const T z = T(0);
+  return fma_(r.d.x, z, fma_(r.d.y, z, r.d.z * z)) == z && r.o.x == r.o.x && r.o.y == r.o.y &&
+         r.o.z == r.o.z;
+}
+
 // reference: include/intersect/intersection.h:17-20
 template <class T> PT_INLINE V3<T> hit_point(const Ray<T> &ray, T t) {
   return ray.o + ray.d * t;

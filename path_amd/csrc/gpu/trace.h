@@ -295,6 +295,8 @@ template <class Stack>
 __device__ __forceinline__ Hit<float>
 trace_closest(const float4 *__restrict__ nodes, const float4 *__restrict__ tris,
               const Ray<float> &ray, float t_limit, float occlude_below, Stack &stack) {
+  if (!ray_can_hit(ray))
+    return {t_limit, kNoHit, 0};
   TraceState ts;
   ts.init(ray, t_limit, occlude_below);
   stack.sp = 0;

@@ -495,7 +495,7 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
         }
         ts.init(ray, shadow ? d.w + 2e-6f : 3.4028235e38f, shadow ? d.w - 2e-6f : -1.0f);
         stack.sp = 0;
-        if (has_nodes)
+        if (has_nodes && ray_can_hit(ray))
           has = true;
         else
           (shadow ? p.st.hit_light : p.st.hit_ext)[slot] = pack_hit(Hit<float>{0.f, kNoHit, 0});
