@@ -663,8 +663,8 @@ def bench_mlp(a, cfg):
 
 
 def mlp_forward_timing(m, iters=20):
-    """Roofline of the dominant inference kernel (k_mlp_forward over 2^20
-    queries) and the layer-by-layer GEMM (training forward) beside it."""
+    """Roofline of the dominant inference kernel (k_mlp_tile over 2^20
+    queries) and the layer-by-layer GEMM beside it."""
     rows_t = 1 << 20
     gemm_ms, fwd_ms = m.time_forward(rows_t, iters)
     gemm_tflops = 2.0 * rows_t * 256 * 256 / (gemm_ms * 1e-3) / 1e12
@@ -675,7 +675,7 @@ def mlp_forward_timing(m, iters=20):
                        "shape": "2^20 x 256 x 256, BF16 in, FP32 accumulate"},
         "roofline": {"bound": "mfma", "achieved": round(fwd_tflops, 2), "peak": 2500.0,
                      "unit": "TFLOP/s", "frac": round(fwd_tflops / 2500.0, 5),
-                     "traffic": None, "kernel": "k_mlp_forward",
+                     "traffic": None, "kernel": "k_mlp_tile",
                      "avg_launch_ms": round(fwd_ms, 4),
                      "flops_per_launch": 2 * rows_t * MLP_MACS,
                      "note": "whole inference forward of 2^20 queries in one kernel "

@@ -52,6 +52,7 @@ SOURCES = [
     "gpu/wavefront.hip",
     "gpu/adjoint.hip",
     "mlp/mlp_kernels.hip",
+    "mlp/mlp_fused.hip",
     "gpu/nrc.hip",
     "gpu/lbvh.hip",
     "gpu/radix_sort.hip",

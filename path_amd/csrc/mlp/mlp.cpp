@@ -69,11 +69,9 @@ bool pt_mlp::init(int dev, uint64_t seed, std::string *err) {
   if (e == hipSuccess)
     e = wbf.ensure(P);
   if (e == hipSuccess)
-    e = launch_to_bf16(w32.ptr, wbf.ptr, P, stream);
+    e = w_frag.ensure(kWFragElems);
   if (e == hipSuccess)
-    e = wbf_t.ensure(P);
-  if (e == hipSuccess)
-    e = launch_transpose_weights(wbf.ptr, wbf_t.ptr, stream);
+    e = wt_frag.ensure(kWtFragElems);
   if (e == hipSuccess)
     e = adam_m.ensure(P);
   if (e == hipSuccess)
@@ -81,9 +79,16 @@ bool pt_mlp::init(int dev, uint64_t seed, std::string *err) {
   if (e == hipSuccess)
     e = grad.ensure(P);
   if (e == hipSuccess)
+    e = out_grad.ensure(size_t(kOut) * kWidth);
+  // outputs 16 .. 31 of the output layer's fragments stay zero
+  if (e == hipSuccess)
+    e = hipMemsetAsync(w_frag.ptr, 0, kWFragElems * sizeof(bf16), stream);
+  if (e == hipSuccess)
     e = hipMemsetAsync(adam_m.ptr, 0, P * 4, stream);
   if (e == hipSuccess)
     e = hipMemsetAsync(adam_v.ptr, 0, P * 4, stream);
+  if (e == hipSuccess && update(kUpdatePack, 0) != PT_OK)
+    e = hipErrorUnknown;
   if (e == hipSuccess)
     e = hipStreamSynchronize(stream);
   if (e != hipSuccess) {
@@ -93,27 +98,15 @@ bool pt_mlp::init(int dev, uint64_t seed, std::string *err) {
   return true;
 }
 
-int pt_mlp::ensure_rows(uint32_t rows_pad, bool training) {
-  HIP_TRY(feat.ensure(size_t(rows_pad) * kFeatures));
-  HIP_TRY(targ.ensure(size_t(rows_pad) * kOut));
-  HIP_TRY(pred.ensure(size_t(rows_pad) * kOutPad));
-  HIP_TRY(x0.ensure(size_t(rows_pad) * kInPad));
-  // inference ping-pongs act[0] / act[1]; training keeps every layer
-  const uint32_t n_act = training ? kHidden : 2;
-  for (uint32_t l = 0; l < n_act; ++l)
-    HIP_TRY(act[l].ensure(size_t(rows_pad) * kWidth));
-  if (training) {
-    HIP_TRY(d_pred.ensure(size_t(rows_pad) * kOutPad));
-    HIP_TRY(g0.ensure(size_t(rows_pad) * kWidth));
-    HIP_TRY(g1.ensure(size_t(rows_pad) * kWidth));
-    HIP_TRY(loss_part.ensure((rows_pad + 255) / 256));
-    HIP_TRY(x0_t.ensure(size_t(rows_pad) * kInPad));
-    for (uint32_t l = 0; l < kHidden; ++l)
-      HIP_TRY(act_t[l].ensure(size_t(rows_pad) * kWidth));
-    HIP_TRY(d_pred_t.ensure(size_t(rows_pad) * kOutPad));
-    HIP_TRY(g0_t.ensure(size_t(rows_pad) * kWidth));
-    HIP_TRY(g1_t.ensure(size_t(rows_pad) * kWidth));
-  }
+int pt_mlp::ensure_training(uint32_t rows_pad, uint32_t steps) {
+  const uint32_t tiles = rows_pad / mlp_tile_rows(rows_pad);
+  HIP_TRY(a_frag.ensure(size_t(kHidden) * rows_pad * kWidth));
+  HIP_TRY(g_frag.ensure(size_t(kHidden) * rows_pad * kWidth));
+  HIP_TRY(masks.ensure(size_t(rows_pad) * (kHidden * kWidth / 32)));
+  HIP_TRY(out_part.ensure(size_t(tiles) * kOut * kWidth));
+  HIP_TRY(loss_part.ensure(tiles));
+  HIP_TRY(split_part.ensure(size_t(kHidden) * mlp_wgrad_splits(rows_pad) * kWidth * kWidth));
+  HIP_TRY(step_losses.ensure(std::max<uint32_t>(steps, 1)));
   return PT_OK;
 }
 
@@ -129,103 +122,98 @@ static GemmArgs gemm_args(const bf16 *A, uint32_t lda, const bf16 *B, uint32_t l
   g.K = K;
   g.C = C;
   g.ldc = ldc;
-  g.k_per_split = (K + 31) / 32 * 32;
   return g;
 }
 
-int pt_mlp::forward_device(const float *d_feat, uint32_t rows_pad, bool training,
-                           hipStream_t on) {
+int pt_mlp::forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad, hipStream_t on) {
   hipStream_t stream = on ? on : this->stream;
-  if (!training && fused_forward) {
-    HIP_TRY(launch_mlp_forward(d_feat, rows_pad, wbf.ptr, pred.ptr, stream));
+  HIP_TRY(pred.ensure(size_t(rows_pad) * kOutPad));
+  if (fused_forward) {
+    MlpTileArgs t{};
+    t.feat = d_feat;
+    t.n = n;
+    t.w_frag = reinterpret_cast<const uint16_t *>(w_frag.ptr);
+    t.pred = pred.ptr;
+    HIP_TRY(launch_mlp_tile(t, rows_pad, false, stream));
     return PT_OK;
   }
-  HIP_TRY(launch_encode(d_feat, rows_pad, x0.ptr, stream));
-  if (training)
-    HIP_TRY(launch_transpose(x0.ptr, rows_pad, kInPad, kInPad, x0_t.ptr, rows_pad, stream));
+  HIP_TRY(x0.ensure(size_t(rows_pad) * kInPad));
+  for (auto &a : act)
+    HIP_TRY(a.ensure(size_t(rows_pad) * kWidth));
+  HIP_TRY(launch_encode(d_feat, n, rows_pad, x0.ptr, stream));
   const bf16 *in = x0.ptr;
   for (uint32_t l = 0; l < kLayers; ++l) {
     const bf16 *w = wbf.ptr + layer_offset(l);
     if (l + 1 < kLayers) {
-      bf16 *out = training ? act[l].ptr : act[l & 1].ptr;
-      GemmArgs g = gemm_args(in, layer_in(l), w, layer_in(l), rows_pad, kWidth, layer_in(l),
-                             out, kWidth);
-      if (training) {
-        g.CT = act_t[l].ptr;
-        g.ldct = rows_pad;
-      }
-      HIP_TRY(launch_gemm(g, false, false, kEpiReluBf16, 1, stream));
+      bf16 *out = act[l & 1].ptr;
+      HIP_TRY(launch_gemm(gemm_args(in, layer_in(l), w, layer_in(l), rows_pad, kWidth,
+                                    layer_in(l), out, kWidth),
+                          kEpiReluBf16, stream));
       in = out;
     } else {
-      GemmArgs g = gemm_args(in, kWidth, w, kWidth, rows_pad, kOutPad, kWidth, pred.ptr,
-                             kOutPad);
-      HIP_TRY(launch_gemm(g, false, false, kEpiF32, 1, stream));
+      HIP_TRY(launch_gemm(gemm_args(in, kWidth, w, kWidth, rows_pad, kOutPad, kWidth, pred.ptr,
+                                    kOutPad),
+                          kEpiF32, stream));
     }
   }
   return PT_OK;
 }
 
-int pt_mlp::backward(uint32_t n, uint32_t rows_pad, float *loss, float *loss_dev) {
-  uint32_t n_part = 0;
-  HIP_TRY(launch_loss(pred.ptr, targ.ptr, n, rows_pad, d_pred.ptr, d_pred_t.ptr, rows_pad,
-                      loss_part.ptr, &n_part, stream));
-  if (loss_dev && n_part)
-    HIP_TRY(launch_loss_sum(loss_part.ptr, n_part, loss_dev, stream));
-  // split-K over the batch for the weight gradients (512 rows per split, at
-  // most 128 splits: 512 workgroups for a 256 x 256 gradient)
-  const uint32_t splits = std::max(1u, std::min(128u, rows_pad / 512u));
-  const uint32_t kps = (rows_pad + splits - 1) / splits;
-  const uint32_t kps32 = (kps + 63) / 64 * 64;
-  HIP_TRY(split_part.ensure(size_t(splits) * kWidth * kWidth));
-  // G: gradient w.r.t. the layer's output [rows x out]; G_t the same
-  // transposed [out x rows]
-  const bf16 *G = d_pred.ptr, *G_t = d_pred_t.ptr;
-  for (int l = int(kLayers) - 1; l >= 0; --l) {
-    const uint32_t in = layer_in(l), out = layer_out(l);
-    const bf16 *a_in_t = l == 0 ? x0_t.ptr : act_t[l - 1].ptr;
-    // dW_l[out x in] = sum over rows of G_t[out][row] a_in_t[in][row]
-    GemmArgs gw = gemm_args(G_t, rows_pad, a_in_t, rows_pad, out, in, rows_pad, split_part.ptr,
-                            in);
-    gw.k_per_split = kps32;
-    const uint32_t used = (rows_pad + kps32 - 1) / kps32;
-    HIP_TRY(launch_gemm(gw, false, false, kEpiSplitF32, used, stream));
-    HIP_TRY(launch_sum_splits(split_part.ptr, used, uint64_t(out) * in,
-                              grad.ptr + layer_offset(l), stream));
-    if (l == 0)
-      break;
-    // dA[rows x in] = (G[rows x out] . W_l[out x in]) masked by the layer
-    // input > 0 (read from its transposed copy, 4 rows per load); W_l^T
-    // ([in][out]) is the B operand; also stored transposed
-    const bool to0 = G != g0.ptr;
-    bf16 *gn = to0 ? g0.ptr : g1.ptr;
-    bf16 *gn_t = to0 ? g0_t.ptr : g1_t.ptr;
-    GemmArgs gd = gemm_args(G, out, wbf_t.ptr + layer_offset(l), out, rows_pad, in, out, gn, in);
-    gd.mask_t = act_t[l - 1].ptr;
-    gd.ldmt = rows_pad;
-    gd.CT = gn_t;
-    gd.ldct = rows_pad;
-    HIP_TRY(launch_gemm(gd, false, false, kEpiMaskBf16, 1, stream));
-    G = gn;
-    G_t = gn_t;
-  }
-  if (loss) {
-    std::vector<float> parts(n_part);
-    HIP_TRY(hipMemcpyAsync(parts.data(), loss_part.ptr, n_part * sizeof(float),
-                           hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
-    double s = 0.0;
-    for (float p : parts)
-      s += p;
-    *loss = float(s);
-  }
+int pt_mlp::gradients(const float *d_feat, const float *d_targ, uint64_t set_rows,
+                      uint64_t seed, uint32_t n, uint32_t rows_pad, float *loss_dev) {
+  MlpTileArgs t{};
+  t.feat = d_feat;
+  t.targ = d_targ;
+  t.set_rows = set_rows;
+  t.seed = seed;
+  t.n = n;
+  t.w_frag = reinterpret_cast<const uint16_t *>(w_frag.ptr);
+  t.wt_frag = reinterpret_cast<const uint16_t *>(wt_frag.ptr);
+  t.a_frag = a_frag.ptr;
+  t.g_frag = g_frag.ptr;
+  t.layer_stride = size_t(rows_pad) * kWidth;
+  t.masks = masks.ptr;
+  t.out_part = out_part.ptr;
+  t.loss_part = loss_part.ptr;
+  HIP_TRY(launch_mlp_tile(t, rows_pad, true, stream));
+  MlpWgradArgs g{};
+  g.a_frag = a_frag.ptr;
+  g.g_frag = g_frag.ptr;
+  g.layer_stride = t.layer_stride;
+  g.rows_pad = rows_pad;
+  g.splits = mlp_wgrad_splits(rows_pad);
+  g.tiles = rows_pad / mlp_tile_rows(rows_pad);
+  g.part = split_part.ptr;
+  g.out_part = out_part.ptr;
+  g.loss_part = loss_part.ptr;
+  g.out_grad = out_grad.ptr;
+  g.loss = loss_dev;
+  HIP_TRY(launch_mlp_wgrad(g, stream));
   return PT_OK;
 }
 
-int pt_mlp::adam(float lr) {
-  ++step;
-  HIP_TRY(launch_adam(w32.ptr, grad.ptr, adam_m.ptr, adam_v.ptr, wbf.ptr, param_count(), lr,
-                      0.9f, 0.99f, 1e-8f, step, stream));
-  HIP_TRY(launch_transpose_weights(wbf.ptr, wbf_t.ptr, stream));
+int pt_mlp::update(int mode, uint32_t rows_pad, float lr) {
+  MlpUpdateArgs u{};
+  u.part = split_part.ptr;
+  u.out_grad = out_grad.ptr;
+  u.splits = mlp_wgrad_splits(rows_pad);
+  u.grad = grad.ptr;
+  u.w = w32.ptr;
+  u.m = adam_m.ptr;
+  u.v = adam_v.ptr;
+  u.w_rows = reinterpret_cast<uint16_t *>(wbf.ptr);
+  u.w_frag = reinterpret_cast<uint16_t *>(w_frag.ptr);
+  u.wt_frag = reinterpret_cast<uint16_t *>(wt_frag.ptr);
+  u.lr = lr;
+  u.beta1 = 0.9f;
+  u.beta2 = 0.99f;
+  u.eps = 1e-8f;
+  if (mode == kUpdateAdam) {
+    ++step;
+    u.c1 = 1.f - powf(u.beta1, float(step));
+    u.c2 = 1.f - powf(u.beta2, float(step));
+  }
+  HIP_TRY(launch_mlp_update(u, mode, stream));
   return PT_OK;
 }
 
@@ -277,8 +265,9 @@ int pt_mlp_set_weights(pt_mlp *m, const float *w) {
     return set_error(PT_ERR_INVALID, "null argument");
   HIP_TRY(hipSetDevice(m->device));
   HIP_TRY(m->w32.upload(w, param_count(), m->stream));
-  HIP_TRY(launch_to_bf16(m->w32.ptr, m->wbf.ptr, param_count(), m->stream));
-  HIP_TRY(launch_transpose_weights(m->wbf.ptr, m->wbf_t.ptr, m->stream));
+  int rc = m->update(kUpdatePack, 0);
+  if (rc != PT_OK)
+    return rc;
   HIP_TRY(hipMemsetAsync(m->adam_m.ptr, 0, param_count() * 4, m->stream));
   HIP_TRY(hipMemsetAsync(m->adam_v.ptr, 0, param_count() * 4, m->stream));
   m->step = 0;
@@ -300,13 +289,8 @@ int pt_mlp_forward(pt_mlp *m, const float *features, uint32_t n, float *out) {
     return PT_OK;
   HIP_TRY(hipSetDevice(m->device));
   const uint32_t rp = mlp_pad_rows(n);
-  int rc = m->ensure_rows(rp, false);
-  if (rc != PT_OK)
-    return rc;
-  HIP_TRY(hipMemsetAsync(m->feat.ptr, 0, size_t(rp) * kFeatures * 4, m->stream));
-  HIP_TRY(hipMemcpyAsync(m->feat.ptr, features, size_t(n) * kFeatures * 4,
-                         hipMemcpyHostToDevice, m->stream));
-  rc = m->forward_device(m->feat.ptr, rp, false);
+  HIP_TRY(m->feat.upload(features, size_t(n) * kFeatures, m->stream));
+  int rc = m->forward_device(m->feat.ptr, n, rp);
   if (rc != PT_OK)
     return rc;
   // compact to n x 3 on the device (reuses the front of the target buffer)
@@ -318,19 +302,17 @@ int pt_mlp_forward(pt_mlp *m, const float *features, uint32_t n, float *out) {
   return PT_OK;
 }
 
-static int load_batch(pt_mlp *m, const float *features, const float *targets, uint32_t n,
-                      uint32_t *rp_out) {
+// Upload a host batch and queue its forward, loss and backward.
+static int batch_gradients(pt_mlp *m, const float *features, const float *targets, uint32_t n,
+                           uint32_t *rp_out) {
   const uint32_t rp = mlp_pad_rows(n);
-  int rc = m->ensure_rows(rp, true);
+  int rc = m->ensure_training(rp, 1);
   if (rc != PT_OK)
     return rc;
-  HIP_TRY(hipMemsetAsync(m->feat.ptr, 0, size_t(rp) * kFeatures * 4, m->stream));
-  HIP_TRY(hipMemcpyAsync(m->feat.ptr, features, size_t(n) * kFeatures * 4,
-                         hipMemcpyHostToDevice, m->stream));
-  HIP_TRY(hipMemcpyAsync(m->targ.ptr, targets, size_t(n) * kOut * 4, hipMemcpyHostToDevice,
-                         m->stream));
+  HIP_TRY(m->feat.upload(features, size_t(n) * kFeatures, m->stream));
+  HIP_TRY(m->targ.upload(targets, size_t(n) * kOut, m->stream));
   *rp_out = rp;
-  return PT_OK;
+  return m->gradients(m->feat.ptr, m->targ.ptr, 0, 0, n, rp, m->step_losses.ptr);
 }
 
 int pt_mlp_gradient(pt_mlp *m, const float *features, const float *targets, uint32_t n,
@@ -339,15 +321,15 @@ int pt_mlp_gradient(pt_mlp *m, const float *features, const float *targets, uint
     return set_error(PT_ERR_INVALID, "null argument or empty batch");
   HIP_TRY(hipSetDevice(m->device));
   uint32_t rp;
-  int rc = load_batch(m, features, targets, n, &rp);
+  int rc = batch_gradients(m, features, targets, n, &rp);
   if (rc == PT_OK)
-    rc = m->forward_device(m->feat.ptr, rp, true);
-  if (rc == PT_OK)
-    rc = m->backward(n, rp, loss);
+    rc = m->update(kUpdateGradient, rp);
   if (rc != PT_OK)
     return rc;
   HIP_TRY(hipMemcpyAsync(grad, m->grad.ptr, param_count() * 4, hipMemcpyDeviceToHost,
                          m->stream));
+  if (loss)
+    HIP_TRY(hipMemcpyAsync(loss, m->step_losses.ptr, 4, hipMemcpyDeviceToHost, m->stream));
   HIP_TRY(hipStreamSynchronize(m->stream));
   return PT_OK;
 }
@@ -358,15 +340,13 @@ int pt_mlp_train_step(pt_mlp *m, const float *features, const float *targets, ui
     return set_error(PT_ERR_INVALID, "null argument or empty batch");
   HIP_TRY(hipSetDevice(m->device));
   uint32_t rp;
-  int rc = load_batch(m, features, targets, n, &rp);
+  int rc = batch_gradients(m, features, targets, n, &rp);
   if (rc == PT_OK)
-    rc = m->forward_device(m->feat.ptr, rp, true);
-  if (rc == PT_OK)
-    rc = m->backward(n, rp, loss);
-  if (rc == PT_OK)
-    rc = m->adam(lr);
+    rc = m->update(kUpdateAdam, rp, lr);
   if (rc != PT_OK)
     return rc;
+  if (loss)
+    HIP_TRY(hipMemcpyAsync(loss, m->step_losses.ptr, 4, hipMemcpyDeviceToHost, m->stream));
   HIP_TRY(hipStreamSynchronize(m->stream));
   return PT_OK;
 }
@@ -380,20 +360,18 @@ int pt_mlp_time_forward(pt_mlp *m, uint32_t rows, uint32_t iters, float *gemm_ms
     return set_error(PT_ERR_INVALID, "null argument or empty workload");
   HIP_TRY(hipSetDevice(m->device));
   const uint32_t rp = mlp_pad_rows(rows);
-  int rc = m->ensure_rows(rp, false);
-  if (rc != PT_OK)
-    return rc;
+  for (auto &a : m->act)
+    HIP_TRY(a.ensure(size_t(rp) * kWidth));
   std::vector<float> f(size_t(rp) * kFeatures, 0.25f);
-  HIP_TRY(hipMemcpyAsync(m->feat.ptr, f.data(), f.size() * 4, hipMemcpyHostToDevice,
-                         m->stream));
-  rc = m->forward_device(m->feat.ptr, rp, false);
+  HIP_TRY(m->feat.upload(f.data(), f.size(), m->stream));
+  int rc = m->forward_device(m->feat.ptr, rp, rp);
   if (rc != PT_OK)
     return rc;
   GemmArgs g = gemm_args(m->act[0].ptr, kWidth, m->wbf.ptr + layer_offset(1), kWidth, rp,
                          kWidth, kWidth, m->act[1].ptr, kWidth);
   HIP_TRY(hipEventRecord(m->ev0, m->stream));
   for (uint32_t i = 0; i < iters; ++i)
-    HIP_TRY(launch_gemm(g, false, false, kEpiReluBf16, 1, m->stream));
+    HIP_TRY(launch_gemm(g, kEpiReluBf16, m->stream));
   HIP_TRY(hipEventRecord(m->ev1, m->stream));
   HIP_TRY(hipEventSynchronize(m->ev1));
   float ms = 0.f;
@@ -402,7 +380,7 @@ int pt_mlp_time_forward(pt_mlp *m, uint32_t rows, uint32_t iters, float *gemm_ms
     *gemm_ms = ms / float(iters);
   HIP_TRY(hipEventRecord(m->ev0, m->stream));
   for (uint32_t i = 0; i < iters && rc == PT_OK; ++i)
-    rc = m->forward_device(m->feat.ptr, rp, false);
+    rc = m->forward_device(m->feat.ptr, rp, rp);
   if (rc != PT_OK)
     return rc;
   HIP_TRY(hipEventRecord(m->ev1, m->stream));
@@ -434,24 +412,15 @@ int pt_mlp_train(pt_mlp *m, uint32_t steps, uint32_t batch, float lr, uint64_t s
     return set_error(PT_ERR_INVALID, "no training set (pt_mlp_set_dataset)");
   HIP_TRY(hipSetDevice(m->device));
   const uint32_t rp = mlp_pad_rows(batch);
-  int rc = m->ensure_rows(rp, true);
+  int rc = m->ensure_training(rp, steps);
   if (rc != PT_OK)
     return rc;
-  HIP_TRY(m->idx.ensure(rp));
-  if (losses)
-    HIP_TRY(m->step_losses.ensure(std::max<uint32_t>(steps, 1)));
-  HIP_TRY(hipMemsetAsync(m->feat.ptr, 0, size_t(rp) * kFeatures * 4, m->stream));
   auto t0 = std::chrono::steady_clock::now();
   for (uint32_t it = 0; it < steps; ++it) {
-    HIP_TRY(launch_random_rows(batch, m->ds_rows, seed + it * 0x632be59bd9b4e019ull,
-                               m->idx.ptr, m->stream));
-    HIP_TRY(launch_gather(m->ds_feat.ptr, m->ds_targ.ptr, m->idx.ptr, batch, m->feat.ptr,
-                          m->targ.ptr, m->stream));
-    rc = m->forward_device(m->feat.ptr, rp, true);
+    rc = m->gradients(m->ds_feat.ptr, m->ds_targ.ptr, m->ds_rows,
+                      seed + it * 0x632be59bd9b4e019ull, batch, rp, m->step_losses.ptr + it);
     if (rc == PT_OK)
-      rc = m->backward(batch, rp, nullptr, losses ? m->step_losses.ptr + it : nullptr);
-    if (rc == PT_OK)
-      rc = m->adam(lr);
+      rc = m->update(kUpdateAdam, rp, lr);
     if (rc != PT_OK)
       return rc;
   }

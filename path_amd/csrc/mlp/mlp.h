@@ -9,20 +9,22 @@ struct pt_mlp {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   uint32_t step = 0; // Adam steps taken
-  bool fused_forward = true; // inference through k_mlp_forward
+  bool fused_forward = true; // inference through k_mlp_tile
 
   pt::host::DeviceBuf<float> w32, adam_m, adam_v, grad;
-  // bf16 weights, and per layer transposed ([in][out]) for the data gradient
-  pt::host::DeviceBuf<pt::mlp::bf16> wbf, wbf_t;
+  // bf16 weights: row-major (the kernels' column order in layer 0) and in the
+  // fused kernels' forward and backward fragment orders
+  pt::host::DeviceBuf<pt::mlp::bf16> wbf, w_frag, wt_frag;
 
   // per-batch buffers (grow-only, rows padded to kRowAlign)
-  pt::host::DeviceBuf<float> feat, targ, pred, loss_part, split_part;
-  pt::host::DeviceBuf<pt::mlp::bf16> x0, act[pt::mlp::kHidden], d_pred, g0, g1;
-  // training: the same tensors transposed ([column][row]), the operands of
-  // the weight-gradient GEMMs, whose K is the batch
-  pt::host::DeviceBuf<pt::mlp::bf16> x0_t, act_t[pt::mlp::kHidden], d_pred_t, g0_t, g1_t;
-  pt::host::DeviceBuf<uint32_t> idx;
-  pt::host::DeviceBuf<float> step_losses; // pt_mlp_train: one mean loss per step
+  pt::host::DeviceBuf<float> feat, targ, pred;
+  pt::host::DeviceBuf<pt::mlp::bf16> x0, act[2]; // layer-by-layer forward
+  // training: layer inputs and output gradients in fragment order, activation
+  // bits, per-tile and per-split partial sums
+  pt::host::DeviceBuf<uint16_t> a_frag, g_frag;
+  pt::host::DeviceBuf<uint32_t> masks;
+  pt::host::DeviceBuf<float> out_part, out_grad, loss_part, split_part;
+  pt::host::DeviceBuf<float> step_losses; // one mean loss per step
 
   // resident training set
   pt::host::DeviceBuf<float> ds_feat, ds_targ;
@@ -30,17 +32,19 @@ struct pt_mlp {
 
   ~pt_mlp();
   bool init(int dev, uint64_t seed, std::string *err);
-  int ensure_rows(uint32_t rows_pad, bool training);
-  // Forward on device features (rows_pad rows, padded rows arbitrary):
-  // pred[rows_pad x 16] fp32. training = keep every layer's activations
-  // (layer-by-layer GEMMs); otherwise the fused kernel unless disabled.
-  int forward_device(const float *d_feat, uint32_t rows_pad, bool training,
+  int ensure_training(uint32_t rows_pad, uint32_t steps);
+  // Forward on device features (n rows; rows up to rows_pad count as zero
+  // features): pred[rows_pad x 16] fp32, by the fused kernel unless disabled.
+  int forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad,
                      hipStream_t on = nullptr);
-  // Loss + backward + gradient into `grad` for the batch already in
-  // feat/targ (n valid rows of rows_pad). The mean loss goes to *loss (host,
-  // synchronising) and/or *loss_dev (device, no synchronisation).
-  int backward(uint32_t n, uint32_t rows_pad, float *loss, float *loss_dev = nullptr);
-  int adam(float lr);
+  // Forward, loss, backward of a batch of n rows: per-split gradients in
+  // split_part / out_grad, the mean loss in *loss_dev (device). With set_rows,
+  // row i is row random(seed, i) of the set_rows rows at d_feat / d_targ.
+  int gradients(const float *d_feat, const float *d_targ, uint64_t set_rows, uint64_t seed,
+                uint32_t n, uint32_t rows_pad, float *loss_dev);
+  // Sum the splits: into `grad`, or into one Adam step; or refresh the bf16
+  // copies of w32 (mlp::MlpUpdate).
+  int update(int mode, uint32_t rows_pad, float lr = 0.f);
 };
 
 namespace pt {

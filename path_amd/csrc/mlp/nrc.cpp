@@ -67,13 +67,7 @@ extern "C" int pt_render_mlp(pt_renderer *r, pt_mlp *m, const pt_scene *scene,
     const uint64_t p1 = std::min(n_pixels, p0 + px_per_chunk);
     const uint32_t rows = uint32_t((p1 - p0) * samples_per);
     const uint32_t rp = mlp_pad_rows(rows);
-    rc = m->ensure_rows(rp, false);
-    if (rc != PT_OK)
-      return rc;
-    HIP_TRY(hipMemsetAsync(m->feat.ptr, 0, size_t(rp) * 9 * sizeof(float), s));
-    HIP_TRY(hipMemcpyAsync(m->feat.ptr, r->nrc_features.ptr + p0 * samples_per * 9,
-                           size_t(rows) * 9 * sizeof(float), hipMemcpyDeviceToDevice, s));
-    rc = m->forward_device(m->feat.ptr, rp, false, s);
+    rc = m->forward_device(r->nrc_features.ptr + p0 * samples_per * 9, rows, rp, s);
     if (rc != PT_OK)
       return rc;
     HIP_TRY(gpu::launch_nrc_combine(r->nrc_base.ptr + p0 * samples_per * 3,
@@ -155,15 +149,7 @@ extern "C" int pt_render_mlp_first_vertex(pt_renderer *r, pt_mlp *m, const pt_sc
     const uint64_t p1 = std::min(n_pixels, p0 + chunk);
     const uint32_t rows = uint32_t(p1 - p0);
     const uint32_t rp = mlp_pad_rows(rows);
-    rc = m->ensure_rows(rp, false);
-    if (rc != PT_OK)
-      return rc;
-    if (rp > rows)
-      HIP_TRY(hipMemsetAsync(m->feat.ptr + size_t(rows) * 9, 0,
-                             size_t(rp - rows) * 9 * sizeof(float), s));
-    HIP_TRY(hipMemcpyAsync(m->feat.ptr, r->nrc_features.ptr + p0 * 9,
-                           size_t(rows) * 9 * sizeof(float), hipMemcpyDeviceToDevice, s));
-    rc = m->forward_device(m->feat.ptr, rp, false, s);
+    rc = m->forward_device(r->nrc_features.ptr + p0 * 9, rows, rp, s);
     if (rc != PT_OK)
       return rc;
     // one "sample" per pixel: out = base + weight * max(pred, 0)

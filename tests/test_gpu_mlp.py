@@ -82,6 +82,46 @@ def test_gradient_matches_reference(net):
         assert e_64 <= 0.15
 
 
+# 32-row tiles below 24,576 rows, 64-row tiles up to 57,344, then 128-row ones;
+# ragged last tiles, and fewer row stages than weight-gradient splits. The bounds are those of
+# test_gradient_matches_reference, from the same roundings.
+@pytest.mark.parametrize("n", [1, 31, 129, 700, 24449, 57300])
+def test_gradient_over_tile_sizes(net, n):
+    from oracle import mlp_ref as M
+    f, t = _data(n, 40 + n)
+    w = net.get_weights()
+    g, loss = net.gradient(f, t)
+    rloss, rg = M.loss_and_grad(w, f, t, emulate=True)
+    assert abs(loss - rloss) <= 1e-3 * rloss
+    offs = np.cumsum([0] + [o * i for o, i in M.SHAPES])
+    for l in range(len(M.SHAPES)):
+        a, b = g[offs[l]:offs[l + 1]], rg[offs[l]:offs[l + 1]]
+        # one sample's gradient has no sum for its roundings to average in
+        assert np.linalg.norm(a - b) <= (3e-2 if n < 32 else 1e-2) * np.linalg.norm(b)
+
+
+def test_train_draws_rows_and_steps_like_train_step(net):
+    """Training on the resident set equals host batches of the rows it draws
+    (SplitMix64 of the row's number), step by step."""
+    f, t = _data(5000, 3)
+    w = net.get_weights()
+    net.set_weights(w)  # Adam from its first step
+    net.set_dataset(f, t)
+    losses, _ = net.train(2, 900, 1e-3, seed=77)
+    trained = net.get_weights()
+    net.set_weights(w)
+    with np.errstate(over="ignore"):
+        for it in range(2):
+            seed = np.uint64(77) + np.uint64(it) * np.uint64(0x632be59bd9b4e019)
+            z = seed + np.uint64(0x9e3779b97f4a7c15) * np.arange(1, 901, dtype=np.uint64)
+            z = (z ^ (z >> np.uint64(30))) * np.uint64(0xbf58476d1ce4e5b9)
+            z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94d049bb133111eb)
+            i = ((z ^ (z >> np.uint64(31))) % np.uint64(5000)).astype(np.int64)
+            assert net.train_step(f[i], t[i], 1e-3) == losses[it]
+    assert np.array_equal(net.get_weights(), trained)
+    net.set_weights(w)
+
+
 def test_training_reduces_loss():
     from path_amd.mlp import RadianceMLP
     m = RadianceMLP(0, seed=5)
