@@ -6,14 +6,22 @@
 namespace pt {
 namespace gpu {
 
-// Counter words used by one render (device memory, zeroed by k_wf_reset).
+// Counter words of one pipeline (device memory, zero at a render's start).
 enum WfCounter : uint32_t {
-  kExtCount = 0,      // entries in the extension-ray queue
-  kShadowCount = 1,   // entries in the shadow-ray queue
-  kExtTotal = 2,      // 64-bit running sum of kExtCount (words 2, 3)
-  kShadowTotal = 4,   // 64-bit running sum of kShadowCount (words 4, 5)
-  kBusyIters = 6,     // iterations that queued at least one ray
+  kExtTotal = 0,      // 64-bit: extension rays queued so far (words 0, 1)
+  kShadowTotal = 2,   // 64-bit: shadow rays queued so far (words 2, 3)
+  kBusyIters = 4,     // iterations that queued at least one ray
+  kIterations = 5,    // iterations traced
   kNumCounters = 8,
+};
+
+// What the host learns of an iteration, in pinned memory: the traversal
+// launch writes it when it starts, so the next iteration is enqueued while it
+// runs.
+struct WfReport {
+  uint32_t ext, shadow; // rays queued
+  uint32_t samples_left; // 0: every sample of this pipeline has been started
+  uint32_t iteration;   // number of the iteration, from 1: written last
 };
 
 // Queue groups. Shade block b belongs to group b % n_groups (n_groups =
@@ -25,11 +33,13 @@ enum WfCounter : uint32_t {
 // all 16k blocks), so one counter per group spreads them over 16 addresses.
 constexpr uint32_t kQueueGroups = 16;
 constexpr uint32_t kGroupStride = 1024; // uint32 words between group counters
+// Odd and even iterations count in sets of their own: while one set is read by
+// its traversal launch, that launch zeroes the other for the next shade step.
 enum GroupCounter : uint32_t {
-  kGroupExt = 0,    // entries in the group's extension-ray segment
-  kGroupShadow = 1, // entries in the group's shadow-ray segment
-  kGroupSample = 2, // 64-bit: samples the group has started
-  kGroupKinds = 3,
+  kGroupExt = 0,    // entries in the group's extension-ray segment (set 0; set 1: + 2)
+  kGroupShadow = 1, // entries in the group's shadow-ray segment (set 0; set 1: + 2)
+  kGroupSample = 4, // 64-bit: samples the group has started
+  kGroupKinds = 5,
 };
 constexpr size_t kGroupCounterWords = size_t(kGroupKinds) * kQueueGroups * kGroupStride;
 
@@ -99,6 +109,9 @@ struct WfParams {
   WfState st;
   WfQueues q;
   uint32_t *counters;       // WfCounter words
+  WfReport *report;         // pinned host memory
+  uint32_t set;             // set of queue counters of this iteration: 0 / 1
+  uint32_t fresh;           // first iteration: every slot is empty, whatever it holds
   uint32_t *group_counters; // GroupCounter words per group (group_counter())
   uint32_t n_groups;        // min(kQueueGroups, shade blocks)
   uint32_t n_shade_blocks;
@@ -113,16 +126,18 @@ struct WfParams {
   uint32_t overflow_stride;           // threads of a traversal launch
 };
 
-// Fold the queue counts of the previous iteration into the running totals and
-// zero them and the group queue counters (one block; safe inside a captured
-// graph).
-hipError_t launch_wf_reset(uint32_t *counters, uint32_t *group_counters, hipStream_t s);
 hipError_t launch_wf_shade(const WfParams &p, bool batched, hipStream_t s);
 // Closest hits of the iteration's extension rays and occlusion of its shadow
-// rays, both queues in one launch; also writes the iteration's queue totals
-// into counters[kExtCount], counters[kShadowCount].
+// rays, both queues in one launch; also adds the iteration's queue counts to
+// the totals, reports them to the host and zeroes the other set of counters.
 hipError_t launch_wf_trace(const WfParams &p, bool batched, uint32_t grid_blocks,
                            hipStream_t s);
+// Takes the paths of the iteration's queues to their ends, each lane tracing
+// its own rays, instead of launch_wf_trace: for an iteration after which few
+// paths and no samples are left.
+constexpr uint32_t kFinishBlockPaths = 64; // queue entries per block and round
+hipError_t launch_wf_finish(const WfParams &p, bool batched, uint32_t grid_blocks,
+                            hipStream_t s);
 // Per-pixel sum of the per-sample radiance in the mega-kernel's order
 // (sequential per thread range, then the lane tree), divided by spp.
 hipError_t launch_wf_reduce(const float *samples, const WorkDivision &wd,

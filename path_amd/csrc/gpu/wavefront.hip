@@ -33,25 +33,9 @@ constexpr uint32_t kFlagLight = 1u << 27;
 constexpr uint32_t kItersMask = 0x00ffffffu;
 } // namespace
 
-__global__ void k_wf_reset(uint32_t *counters, uint32_t *group_counters) {
-  const uint32_t t = threadIdx.x;
-  if (t < 2 * kQueueGroups)
-    *group_counter(group_counters, t < kQueueGroups ? kGroupExt : kGroupShadow,
-                   t % kQueueGroups) = 0;
-  if (t != 0)
-    return;
-  const uint32_t ne = counters[kExtCount], ns = counters[kShadowCount];
-  auto *tot = reinterpret_cast<unsigned long long *>(counters);
-  tot[kExtTotal / 2] += ne;
-  tot[kShadowTotal / 2] += ns;
-  counters[kBusyIters] += (ne + ns) != 0u;
-  counters[kExtCount] = 0;
-  counters[kShadowCount] = 0;
-}
-
-hipError_t launch_wf_reset(uint32_t *counters, uint32_t *group_counters, hipStream_t s) {
-  hipLaunchKernelGGL(k_wf_reset, dim3(1), dim3(64), 0, s, counters, group_counters);
-  return hipGetLastError();
+// Counter of group g in this iteration's set.
+__device__ __forceinline__ uint32_t *queue_counter(const WfParams &p, uint32_t kind, uint32_t g) {
+  return group_counter(p.group_counters, kind + 2u * p.set, g);
 }
 
 // Samples are dealt to the groups in chunks of kSampleChunk consecutive
@@ -153,12 +137,59 @@ __device__ __forceinline__ uint32_t find_scene(const WfBatch &b,
   return lo;
 }
 
+// State of the path in `slot`. The light multiplier exists only while a light
+// sample is pending, the continuation direction only while the path continues.
+__device__ __forceinline__ PathState<float> load_path(const WfParams &p, uint32_t slot,
+                                                      uint32_t flags, Ray<float> *last) {
+  const float4 m = p.st.mult[slot];
+  const F3 lm = (flags & kFlagLight) ? p.st.light[slot] : F3{0.f, 0.f, 0.f};
+  const F3 tot = p.st.total[slot];
+  const F3 o = p.st.origin[slot];
+  const F3 d = (flags & kFlagHasNext) ? p.st.dir[slot] : o;
+  PathState<float> st;
+  st.iters = flags & kItersMask;
+  st.count_emission = (flags & kFlagCountEmission) ? 1u : 0u;
+  st.has_next = (flags & kFlagHasNext) ? 1u : 0u;
+  st.n_light = (flags & kFlagLight) ? 1u : 0u;
+  st.ray_has_target = 0;
+  st.ray_target = 0.f;
+  st.ray_mult = {m.x, m.y, m.z};
+  st.light_target = m.w;
+  st.light_mult = {lm.x, lm.y, lm.z};
+  st.total = {tot.x, tot.y, tot.z};
+  *last = {{o.x, o.y, o.z}, {d.x, d.y, d.z}};
+  return st;
+}
+
+// First-hit surface of a pixel.
+__device__ __forceinline__ void write_gbuffer(const WfParams &p, const SlotScene &sc,
+                                              uint32_t location, const VertexInfo<float> &vi) {
+  const Material<float> &mat = sc.view.materials[vi.material];
+  V3<float> alb = material_albedo(mat);
+  float *g = p.gbuffer + 12 * size_t(sc.pixel_off + location);
+  g[0] = vi.p.x, g[1] = vi.p.y, g[2] = vi.p.z;
+  g[3] = vi.normal.x, g[4] = vi.normal.y, g[5] = vi.normal.z;
+  g[6] = alb.x, g[7] = alb.y, g[8] = alb.z;
+  g[9] = mat.emission.x, g[10] = mat.emission.y, g[11] = mat.emission.z;
+}
+
+// Radiance of a finished path.
+__device__ __forceinline__ void write_sample(const WfParams &p, const SlotScene &sc,
+                                             uint32_t location, uint32_t sample,
+                                             V3<float> radiance) {
+  float *out =
+      p.out_samples + 3 * (size_t(sc.pixel_off + location) * p.rng.samples_per + sample);
+  out[0] = radiance.x;
+  out[1] = radiance.y;
+  out[2] = radiance.z;
+}
+
 template <class R, bool kBatch>
 __device__ __forceinline__ void wf_shade(const WfParams &p) {
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t group = blockIdx.x % p.n_groups;
   const bool in_range = slot < p.n_slots;
-  uint4 meta = in_range ? p.st.meta[slot] : make_uint4(0, 0, 0, 0);
+  uint4 meta = in_range && !p.fresh ? p.st.meta[slot] : make_uint4(0, 0, 0, 0);
   bool active = in_range && (meta.w & kFlagActive);
   uint32_t scene = 0;
   if (kBatch && active)
@@ -171,35 +202,18 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
   float light_target = 0.f;
   PathState<float> ns;
   uint32_t location = meta.x, sample = meta.y, counter = meta.z;
-  // Fields that a step leaves unchanged are neither re-read nor re-written:
-  // the light multiplier exists only while a light sample is pending, the
-  // continuation direction only while the path continues, and the radiance
+  // Fields that a step leaves unchanged are not re-written: the radiance
   // total is stored only when it changed.
   bool total_dirty = false;
   if (active) {
     SlotScene sc = slot_scene<kBatch>(p, scene);
-    float4 m = p.st.mult[slot];
-    const F3 lm = (meta.w & kFlagLight) ? p.st.light[slot] : F3{0.f, 0.f, 0.f};
-    const F3 tot = p.st.total[slot];
-    const F3 o = p.st.origin[slot];
-    const F3 d = (meta.w & kFlagHasNext) ? p.st.dir[slot] : o;
-    PathState<float> st;
-    st.iters = meta.w & kItersMask;
-    st.count_emission = (meta.w & kFlagCountEmission) ? 1u : 0u;
-    st.has_next = (meta.w & kFlagHasNext) ? 1u : 0u;
-    st.n_light = (meta.w & kFlagLight) ? 1u : 0u;
-    st.ray_has_target = 0;
-    st.ray_target = 0.f;
-    st.ray_mult = {m.x, m.y, m.z};
-    st.light_target = m.w;
-    st.light_mult = {lm.x, lm.y, lm.z};
-    st.total = {tot.x, tot.y, tot.z};
+    Ray<float> last;
+    const PathState<float> st = load_path(p, slot, meta.w, &last);
     Hit<float> light_hit = {0.f, kNoHit, 0}, next_hit = {0.f, kNoHit, 0};
     if (st.n_light)
       light_hit = unpack_hit(p.st.hit_light[slot]);
     if (st.has_next)
       next_hit = unpack_hit(p.st.hit_ext[slot]);
-    Ray<float> last = {{o.x, o.y, o.z}, {d.x, d.y, d.z}};
     R rng = make_rng<R>(p.rng, location, sample, counter);
     Ray<float> nl = last, nn = last;
     // The vertex record is always filled (a few register moves): a pointer
@@ -210,23 +224,13 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
     const bool want_gbuffer = p.gbuffer && st.iters == 0 && sample == 0;
     finished = rendering_equation_iteration(st, rng, last, light_hit, next_hit,
                                             p.settings, sc.view, &ns, &nl, &nn, &vi);
-    if (want_gbuffer && vi.valid) {
-      const Material<float> &mat = sc.view.materials[vi.material];
-      V3<float> alb = material_albedo(mat);
-      float *g = p.gbuffer + 12 * size_t(sc.pixel_off + location);
-      g[0] = vi.p.x, g[1] = vi.p.y, g[2] = vi.p.z;
-      g[3] = vi.normal.x, g[4] = vi.normal.y, g[5] = vi.normal.z;
-      g[6] = alb.x, g[7] = alb.y, g[8] = alb.z;
-      g[9] = mat.emission.x, g[10] = mat.emission.y, g[11] = mat.emission.z;
-    }
+    if (want_gbuffer && vi.valid)
+      write_gbuffer(p, sc, location, vi);
     counter = rng_counter(rng);
-    total_dirty = ns.total.x != tot.x || ns.total.y != tot.y || ns.total.z != tot.z;
+    total_dirty =
+        ns.total.x != st.total.x || ns.total.y != st.total.y || ns.total.z != st.total.z;
     if (finished) {
-      float *out = p.out_samples +
-                   3 * (size_t(sc.pixel_off + location) * p.rng.samples_per + sample);
-      out[0] = ns.total.x;
-      out[1] = ns.total.y;
-      out[2] = ns.total.z;
+      write_sample(p, sc, location, sample, ns.total);
     } else {
       if (ns.n_light) {
         push_light = true;
@@ -317,8 +321,8 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
     if (push_light)
       p.st.light_dir[slot] =
           make_float4(light_d.x, light_d.y, light_d.z, light_target);
-  } else if (in_range && (active || want_new)) {
-    p.st.meta[slot] = make_uint4(0, 0, 0, 0); // empty slot
+  } else if (in_range && (active || p.fresh)) {
+    p.st.meta[slot] = make_uint4(0, 0, 0, 0); // the slot has become empty
   }
 
   // ---- append rays to the queues (order within the block: wave, lane) ----
@@ -333,9 +337,9 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
   if (threadIdx.x == 0) {
     uint32_t te = s_counts[1][0] + s_counts[1][1] + s_counts[1][2] + s_counts[1][3];
     uint32_t ts = s_counts[2][0] + s_counts[2][1] + s_counts[2][2] + s_counts[2][3];
-    s_queue_base[0] = te ? atomicAdd(group_counter(p.group_counters, kGroupExt, group), te) : 0u;
+    s_queue_base[0] = te ? atomicAdd(queue_counter(p, kGroupExt, group), te) : 0u;
     s_queue_base[1] =
-        ts ? atomicAdd(group_counter(p.group_counters, kGroupShadow, group), ts) : 0u;
+        ts ? atomicAdd(queue_counter(p, kGroupShadow, group), ts) : 0u;
   }
   __syncthreads();
   uint32_t be = s_queue_base[0], bs = s_queue_base[1];
@@ -414,6 +418,39 @@ constexpr uint32_t kRefillMinIdle = 16;
 // batched scenes: no difference between 3 and 4); refill thresholds 8 / 16 /
 // 24 / 32: 884 / 895-898 / 899-900 / 887.
 constexpr uint32_t kTraceVote = 4;
+// Wave 0 of a block: s_prefix[g] = first entry of segment g of the
+// concatenated queues (extension segments, then shadow segments). Returns the
+// lane's inclusive sum.
+__device__ __forceinline__ uint32_t scan_queues(const WfParams &p, uint32_t *s_prefix) {
+  const uint32_t g = threadIdx.x;
+  uint32_t sum =
+      g < 2 * kQueueGroups
+          ? *queue_counter(p, g < kQueueGroups ? kGroupExt : kGroupShadow, g % kQueueGroups)
+          : 0u;
+#pragma unroll
+  for (uint32_t off = 1; off < 2 * kQueueGroups; off <<= 1) {
+    const uint32_t v = __shfl_up(sum, off, 64);
+    sum += g >= off ? v : 0u;
+  }
+  if (g < 2 * kQueueGroups)
+    s_prefix[g + 1] = sum;
+  if (g == 0)
+    s_prefix[0] = 0;
+  return sum;
+}
+
+// Slot at entry v of the concatenated queues.
+__device__ __forceinline__ uint32_t queue_slot(const WfParams &p, const uint32_t *s_prefix,
+                                               uint32_t v, bool *shadow) {
+  uint32_t g = 0;
+  for (uint32_t step = kQueueGroups; step; step >>= 1)
+    if (s_prefix[g + step] <= v)
+      g += step;
+  *shadow = g >= kQueueGroups;
+  const uint32_t *q = *shadow ? p.q.shadow : p.q.ext;
+  return q[size_t(g % kQueueGroups) * p.q.group_cap + (v - s_prefix[g])];
+}
+
 // Both queues of an iteration in one launch (the extension segments, then
 // the shadow segments, concatenated); a lane's entry decides its ray kind (a shadow ray carries its target window and stops at the first
 // occluder). One launch instead of an extension launch followed by a shadow
@@ -424,17 +461,35 @@ template <bool kBatch>
 __device__ __forceinline__ void wf_trace(const WfParams &p) {
   __shared__ int lds_stack[kLdsStackInts * 4];
   __shared__ uint32_t s_prefix[2 * kQueueGroups + 1];
-  if (threadIdx.x == 0) {
-    uint32_t sum = 0;
-    for (uint32_t g = 0; g < 2 * kQueueGroups; ++g) {
-      s_prefix[g] = sum;
-      sum += *group_counter(p.group_counters, g < kQueueGroups ? kGroupExt : kGroupShadow,
-                            g % kQueueGroups);
-    }
-    s_prefix[2 * kQueueGroups] = sum;
+  if (threadIdx.x < 64) {
+    const uint32_t g = threadIdx.x, sum = scan_queues(p, s_prefix);
     if (blockIdx.x == 0) {
-      p.counters[kExtCount] = s_prefix[kQueueGroups];
-      p.counters[kShadowCount] = sum - s_prefix[kQueueGroups];
+      if (g < 2 * kQueueGroups)
+        *group_counter(p.group_counters,
+                       (g < kQueueGroups ? kGroupExt : kGroupShadow) + 2u * (p.set ^ 1u),
+                       g % kQueueGroups) = 0;
+      const bool left =
+          g < p.n_groups && *reinterpret_cast<const unsigned long long *>(group_counter(
+                                p.group_counters, kGroupSample, g)) < group_sample_count(p, g);
+      const uint32_t any_left = __ballot(left) != 0;
+      const uint32_t ne = __shfl(sum, kQueueGroups - 1, 64);
+      const uint32_t ns = __shfl(sum, 2 * kQueueGroups - 1, 64) - ne;
+      if (g == 0) {
+        auto *tot = reinterpret_cast<unsigned long long *>(p.counters);
+        tot[kExtTotal / 2] += ne;
+        tot[kShadowTotal / 2] += ns;
+        p.counters[kBusyIters] += ne + ns != 0u;
+        const uint32_t it = ++p.counters[kIterations];
+        auto tell = [](uint32_t *at, uint32_t v, int order) {
+          order == __ATOMIC_RELEASE
+              ? __hip_atomic_store(at, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM)
+              : __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        };
+        tell(&p.report->ext, ne, __ATOMIC_RELAXED);
+        tell(&p.report->shadow, ns, __ATOMIC_RELAXED);
+        tell(&p.report->samples_left, any_left, __ATOMIC_RELAXED);
+        tell(&p.report->iteration, it, __ATOMIC_RELEASE);
+      }
     }
   }
   __syncthreads();
@@ -470,13 +525,7 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
       if (!has && next + pre < end) {
         const uint32_t j = next + pre;
         const uint32_t v = j < e_len ? e0 + j : n_ext + s0 + (j - e_len);
-        uint32_t g = 0;
-        for (uint32_t step = kQueueGroups; step; step >>= 1)
-          if (s_prefix[g + step] <= v)
-            g += step;
-        shadow = g >= kQueueGroups;
-        const uint32_t *q = shadow ? p.q.shadow : p.q.ext;
-        slot = q[size_t(g % kQueueGroups) * p.q.group_cap + (v - s_prefix[g])];
+        slot = queue_slot(p, s_prefix, v, &shadow);
         const F3 o = p.st.origin[slot];
         float4 d;
         if (shadow) {
@@ -530,6 +579,112 @@ hipError_t launch_wf_trace(const WfParams &p, bool batched, uint32_t grid_blocks
     hipLaunchKernelGGL((k_wf_trace<true>), dim3(grid_blocks), dim3(256), 0, s, p);
   else
     hipLaunchKernelGGL((k_wf_trace<false>), dim3(grid_blocks), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+
+// The paths of the iteration's queues, each taken to its end by one lane that
+// traces its own rays: a render's last iterations have few rays, and each costs
+// two launches and the latency of its longest ray whatever their number. Only
+// kFinishLanes lanes of a wave take a path, so that few paths still spread over
+// the chip and wait for few others' rays. The vertices are those of wf_shade,
+// so the results are the same bits.
+constexpr uint32_t kFinishLanes = kFinishBlockPaths / 4;
+
+template <class R, bool kBatch>
+__global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
+  __shared__ int lds_stack[kLdsStackInts * 4];
+  __shared__ uint32_t s_prefix[2 * kQueueGroups + 1];
+  if (threadIdx.x < 64)
+    scan_queues(p, s_prefix);
+  __syncthreads();
+  const uint32_t total = s_prefix[2 * kQueueGroups];
+  const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+  const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
+  LdsStack stack{lds_stack_column(lds_stack), p.stack_overflow + gtid, p.overflow_stride};
+  uint32_t n_ext = 0, n_shadow = 0;
+  for (uint32_t v = (gtid >> 6) * kFinishLanes + lane; v < total && lane < kFinishLanes;
+       v += n_waves * kFinishLanes) {
+    bool shadow;
+    const uint32_t slot = queue_slot(p, s_prefix, v, &shadow);
+    const uint4 meta = p.st.meta[slot];
+    if (shadow && (meta.w & kFlagHasNext))
+      continue; // its extension ray's entry takes the path
+    const uint32_t location = meta.x, sample = meta.y;
+    const uint32_t scene = kBatch ? p.st.scene[slot] : 0u;
+    const SlotScene sc = slot_scene<kBatch>(p, scene);
+    const float4 *nodes = p.scene.nodes, *tris = p.scene.tris;
+    bool has_nodes = true;
+    if constexpr (kBatch) {
+      const SceneDesc &sd = p.batch.scenes[scene];
+      nodes = p.batch.nodes + kNodeFloat4 * size_t(sd.node_off);
+      tris = p.batch.tris + 3 * size_t(sd.tri_off);
+      has_nodes = sd.has_nodes != 0;
+    }
+    Ray<float> last;
+    PathState<float> st = load_path(p, slot, meta.w, &last);
+    Ray<float> light_ray = last;
+    if (st.n_light) {
+      const float4 d = p.st.light_dir[slot];
+      light_ray.d = {d.x, d.y, d.z};
+    }
+    R rng = make_rng<R>(p.rng, location, sample, meta.z);
+    for (;;) {
+      Hit<float> light_hit = {0.f, kNoHit, 0}, next_hit = {0.f, kNoHit, 0};
+      if (st.n_light) {
+        ++n_shadow;
+        if (has_nodes)
+          light_hit = trace_closest(nodes, tris, light_ray, st.light_target + 2e-6f,
+                                    st.light_target - 2e-6f, stack);
+      }
+      if (st.has_next) {
+        ++n_ext;
+        if (has_nodes)
+          next_hit = trace_closest(nodes, tris, last, 3.4028235e38f, -1.0f, stack);
+      }
+      PathState<float> ns;
+      Ray<float> nl = light_ray, nn = last;
+      VertexInfo<float> vi;
+      vi.valid = 0u;
+      const bool done = rendering_equation_iteration(st, rng, last, light_hit, next_hit,
+                                                     p.settings, sc.view, &ns, &nl, &nn, &vi);
+      if (p.gbuffer && st.iters == 0 && sample == 0 && vi.valid)
+        write_gbuffer(p, sc, location, vi);
+      if (done) {
+        write_sample(p, sc, location, sample, ns.total);
+        break;
+      }
+      st = ns;
+      light_ray = nl;
+      last = nn;
+    }
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    n_ext += __shfl_xor(n_ext, off, 64);
+    n_shadow += __shfl_xor(n_shadow, off, 64);
+  }
+  if (lane == 0 && n_ext + n_shadow) {
+    auto *tot = reinterpret_cast<unsigned long long *>(p.counters);
+    atomicAdd(tot + kExtTotal / 2, (unsigned long long)n_ext);
+    atomicAdd(tot + kShadowTotal / 2, (unsigned long long)n_shadow);
+    if (gtid == 0)
+      atomicAdd(p.counters + kBusyIters, 1u);
+  }
+}
+
+hipError_t launch_wf_finish(const WfParams &p, bool batched, uint32_t grid_blocks,
+                            hipStream_t s) {
+  if (grid_blocks == 0 || uint64_t(grid_blocks) * 256 > p.overflow_stride)
+    return hipErrorInvalidValue;
+  const dim3 grid(grid_blocks), block(256);
+  const bool sobol = p.rng.type == kRngSobel;
+  if (batched && sobol)
+    hipLaunchKernelGGL((k_wf_finish<TableRng, true>), grid, block, 0, s, p);
+  else if (batched)
+    hipLaunchKernelGGL((k_wf_finish<HashRng, true>), grid, block, 0, s, p);
+  else if (sobol)
+    hipLaunchKernelGGL((k_wf_finish<TableRng, false>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((k_wf_finish<HashRng, false>), grid, block, 0, s, p);
   return hipGetLastError();
 }
 

@@ -134,8 +134,8 @@ pt_renderer::~pt_renderer() {
     for (hipEvent_t e : pipe)
       if (e)
         (void)hipEventDestroy(e);
-  if (wf_host_counts)
-    (void)hipHostFree(wf_host_counts);
+  if (wf_reports)
+    (void)hipHostFree(wf_reports);
   for (hipStream_t ps : pipe_streams)
     if (ps)
       (void)hipStreamDestroy(ps);

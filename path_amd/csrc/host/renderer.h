@@ -175,7 +175,9 @@ struct pt_renderer {
   int device = 0;
   hipStream_t stream = nullptr;   // everything, and wavefront pipeline 0
   hipStream_t pipe_streams[kMaxPipes - 1] = {}; // wavefront pipelines 1..
-  uint32_t n_pipes = 3; // wavefront pipelines of a render (1..kMaxPipes)
+  // wavefront pipelines of a render (1..kMaxPipes); 0: three, fewer for pools
+  // of few paths (wavefront_alloc)
+  uint32_t n_pipes = 0;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr, ev_fork = nullptr;
   pt_render_stats stats{};
   bool profiling = false;
@@ -208,10 +210,9 @@ struct pt_renderer {
   pt::host::DeviceBuf<uint32_t> wf_q_ext, wf_q_shadow;
   pt::host::DeviceBuf<int> wf_stack_overflow;
   pt::host::DeviceBuf<uint32_t> wf_counters;
-  pt::host::DeviceBuf<uint32_t> wf_group_counters;
   pt::host::DeviceBuf<float> wf_samples;
   pt::host::DeviceBuf<uint32_t> wf_scene;
-  uint32_t *wf_host_counts = nullptr; // pinned
+  pt::gpu::WfReport *wf_reports = nullptr; // pinned, one per pipeline
 
   // batched-render buffers (concatenated scenes)
   pt::host::DeviceBuf<pt::host::GpuNode> b_nodes;

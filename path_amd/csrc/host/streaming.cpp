@@ -26,6 +26,29 @@ using namespace pt::host;
 namespace pt {
 namespace host {
 
+// Paths that make a pipeline of their own worth its host thread, stream and
+// launches: 16,384 samples of a 20,516-triangle scene 1,193 -> 799 us and of
+// the 36-triangle box 452 -> 265 with one pipeline, 1.0 M samples of a
+// 5,156-triangle scene 1,152 with three and 1,657 with one (2^16 / 2^18 / 2^19
+// paths per pipeline, 0.25 M samples of that scene: 1,769 / 1,808 / 1,808).
+constexpr uint32_t kMinPipeSlots = 1u << 18;
+
+// Rays queued by an iteration after which the remaining paths are finished by
+// one launch (k_wf_finish). 988,317 samples of the 36-triangle box with
+// roulette (28 iterations), never / 2,048 / 8,192 / 32,768 / 131,072 rays: 1,197 /
+// 1,051 / 999 / 928 / 959 us; 82k triangles, 16.8 M samples: no difference. The
+// limit keeps a small render's first vertices (16,384 paths, 20,516 triangles:
+// 771 us, 895 when finished from there) in the shared queues.
+constexpr uint32_t kFinishRays = 12288;
+
+// Counters of the first n pipelines: every pipeline's WfCounter words (padded
+// to a group counter's 4 KB), then the group counters, in one buffer that one
+// fill clears.
+static size_t counter_words(int n) {
+  static_assert(kMaxPipes * gpu::kNumCounters <= gpu::kGroupStride);
+  return gpu::kGroupStride + size_t(n) * gpu::kGroupCounterWords;
+}
+
 int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
                     uint32_t n_slots, uint64_t total_samples, bool batched,
                     uint32_t trace_blocks) {
@@ -41,10 +64,13 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
   if (batched)
     HIP_TRY(r.wf_scene.ensure(n_slots));
   HIP_TRY(r.wf_samples.ensure(size_t(total_samples) * 3));
-  // r.n_pipes pipelines (an equal share of the slots each, their own stream,
-  // queues and counters) while each gets at least one shade block: the
-  // memory-bound shade step of one overlaps the ALU-bound traversal of another.
-  w.n = int(std::max(1u, std::min({r.n_pipes, uint32_t(kMaxPipes), n_slots / 256})));
+  // Pipelines have an equal share of the slots each, their own stream, queues
+  // and counters: the memory-bound shade step of one overlaps the ALU-bound
+  // traversal of another.
+  // A given number of pipelines is kept to one shade block each.
+  const uint32_t pipes = r.n_pipes ? std::min(r.n_pipes, n_slots / 256)
+                                   : std::min(3u, n_slots / kMinPipeSlots);
+  w.n = int(std::max(1u, std::min(pipes, uint32_t(kMaxPipes))));
   uint32_t first[kMaxPipes + 1] = {0};
   for (int h = 0; h < w.n; ++h) {
     const uint32_t left = n_slots - first[h], pipes_left = uint32_t(w.n - h);
@@ -63,8 +89,7 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
   }
   HIP_TRY(r.wf_q_ext.ensure(queue_total));
   HIP_TRY(r.wf_q_shadow.ensure(queue_total));
-  HIP_TRY(r.wf_counters.ensure(size_t(kMaxPipes) * gpu::kNumCounters));
-  HIP_TRY(r.wf_group_counters.ensure(size_t(kMaxPipes) * gpu::kGroupCounterWords));
+  HIP_TRY(r.wf_counters.ensure(counter_words(kMaxPipes)));
   const uint32_t trace_threads = trace_blocks * 256;
   HIP_TRY(r.wf_stack_overflow.ensure(size_t(kMaxPipes) * gpu::kOverflowDepth * trace_threads));
   size_t queue_off = 0;
@@ -82,7 +107,7 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
     p.q = {r.wf_q_ext.ptr + queue_off, r.wf_q_shadow.ptr + queue_off, caps[h]};
     queue_off += size_t(caps[h]) * groups[h];
     p.counters = r.wf_counters.ptr + size_t(h) * gpu::kNumCounters;
-    p.group_counters = r.wf_group_counters.ptr + size_t(h) * gpu::kGroupCounterWords;
+    p.group_counters = r.wf_counters.ptr + counter_words(0) + size_t(h) * gpu::kGroupCounterWords;
     p.n_groups = groups[h];
     p.n_shade_blocks = (p.n_slots + 255) / 256;
     p.group_base = group_base;
@@ -95,55 +120,81 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
   return PT_OK;
 }
 
-// Enqueue one iteration of one pipeline: fold the previous queue counts into
-// the totals and zero them, shade, trace the extension and shadow rays (one
-// launch), copy the counts to pinned host memory.
-static hipError_t enqueue_iteration(pt_renderer &r, const gpu::WfParams &p, int pipe,
-                                    bool batched, uint32_t trace_blocks,
-                                    bool profile_events) {
+// Enqueue iteration number `iter` (from 0) of one pipeline: shade, then trace
+// the extension and shadow rays (one launch, which also reports the queues'
+// sizes to the host), or, with finish_blocks, take its paths to their ends.
+static hipError_t enqueue_iteration(pt_renderer &r, gpu::WfParams &p, int pipe, uint64_t iter,
+                                    bool batched, uint32_t trace_blocks, bool graph,
+                                    bool profile_events, uint32_t finish_blocks = 0) {
   hipStream_t s = r.pipe_stream(pipe);
   hipEvent_t *ev = r.ev_prof[pipe];
   hipError_t e;
-  if ((e = gpu::launch_wf_reset(p.counters, p.group_counters, s)) != hipSuccess)
-    return e;
+  p.set = uint32_t(iter & 1);
+  p.fresh = iter == 0 && !graph;
   if ((e = gpu::launch_wf_shade(p, batched, s)) != hipSuccess)
     return e;
   if (profile_events && (e = hipEventRecord(ev[0], s)) != hipSuccess)
     return e;
-  if ((e = gpu::launch_wf_trace(p, batched, trace_blocks, s)) != hipSuccess)
+  e = finish_blocks ? gpu::launch_wf_finish(p, batched, finish_blocks, s)
+                    : gpu::launch_wf_trace(p, batched, trace_blocks, s);
+  if (e != hipSuccess)
     return e;
   if (profile_events && (e = hipEventRecord(ev[1], s)) != hipSuccess)
     return e;
-  // queue totals of this iteration (written by the extension trace)
-  return hipMemcpyAsync(r.wf_host_counts + size_t(pipe) * gpu::kNumCounters, p.counters,
-                        sizeof(uint32_t) * gpu::kNumCounters, hipMemcpyDeviceToHost, s);
+  return hipSuccess;
+}
+
+// Wait until the pipeline has reported iteration `iteration` (numbered from
+// 1): its traversal has started. The stream is asked now and then, so that a
+// failed launch ends the wait.
+static hipError_t wait_report(const volatile gpu::WfReport *rep, uint32_t iteration,
+                              hipStream_t s) {
+  auto there = [&] {
+    return int32_t(__atomic_load_n(&rep->iteration, __ATOMIC_ACQUIRE) - iteration) >= 0;
+  };
+  for (uint32_t spin = 1; !there(); ++spin) {
+    __builtin_ia32_pause();
+    if (spin % 8192 != 0)
+      continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady)
+      continue;
+    if (e != hipSuccess)
+      return e;
+    return there() ? hipSuccess : hipErrorUnknown; // drained: it has been written, or never will
+  }
+  return hipSuccess;
 }
 
 int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_blocks,
                   uint32_t iters_per_sync) {
   hipStream_t s0 = r.stream;
+  const bool prof = r.profiling;
+  const bool use_graph = r.use_graphs && !prof;
+  HIP_TRY(hipMemsetAsync(r.wf_counters.ptr, 0, sizeof(uint32_t) * counter_words(w.n), s0));
+  if (use_graph) // its iterations are all alike, so empty slots have to say so
+    for (int h = 0; h < w.n; ++h)
+      HIP_TRY(hipMemsetAsync(w.p[h].st.meta, 0, size_t(w.p[h].n_slots) * sizeof(uint4), s0));
+  if (!r.wf_reports)
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r.wf_reports),
+                          sizeof(gpu::WfReport) * kMaxPipes, hipHostMallocDefault));
   for (int h = 0; h < w.n; ++h) {
-    const gpu::WfParams &p = w.p[h];
-    HIP_TRY(hipMemsetAsync(p.st.meta, 0, size_t(p.n_slots) * sizeof(uint4), s0));
-    HIP_TRY(hipMemsetAsync(p.group_counters, 0, sizeof(uint32_t) * gpu::kGroupCounterWords, s0));
-    HIP_TRY(hipMemsetAsync(p.counters, 0, sizeof(uint32_t) * gpu::kNumCounters, s0));
+    r.wf_reports[h] = gpu::WfReport{};
+    w.p[h].report = r.wf_reports + h;
   }
-  if (!r.wf_host_counts)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r.wf_host_counts),
-                          sizeof(uint32_t) * kMaxPipes * gpu::kNumCounters,
-                          hipHostMallocDefault));
   // the other pipelines start after everything enqueued so far on stream 0
   // (scene upload, state clears)
   HIP_TRY(hipEventRecord(r.ev_fork, s0));
   for (int h = 1; h < w.n; ++h)
     HIP_TRY(hipStreamWaitEvent(r.pipe_stream(h), r.ev_fork, 0));
-  const bool prof = r.profiling;
   if (iters_per_sync == 0)
     iters_per_sync = 1;
   // Profiling needs per-iteration event reads, so it syncs every iteration.
   if (prof)
     iters_per_sync = 1;
-  const bool use_graph = r.use_graphs && !prof;
+  // a graph holds whole pairs of iterations (the two sets of queue counters)
+  if (use_graph)
+    iters_per_sync += iters_per_sync & 1u;
   // Each pipeline runs its own host loop (pipelines 1.. on host threads of
   // their own), so the pipelines drift apart and one's shade step overlaps
   // another's traversal instead of running in lockstep.
@@ -166,7 +217,7 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
       hipGraph_t graph = nullptr;
       hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
       for (uint32_t k = 0; k < iters_per_sync && e == hipSuccess; ++k)
-        e = enqueue_iteration(r, w.p[h], h, batched, trace_blocks, false);
+        e = enqueue_iteration(r, w.p[h], h, k, batched, trace_blocks, true, false);
       hipError_t e2 = hipStreamEndCapture(s, &graph);
       if (e == hipSuccess && e2 == hipSuccess)
         e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -186,20 +237,24 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
         out.launches += iters_per_sync;
       } else {
         for (uint32_t k = 0; k < iters_per_sync && out.err == hipSuccess; ++k) {
-          out.err = enqueue_iteration(r, w.p[h], h, batched, trace_blocks, prof);
+          out.err = enqueue_iteration(r, w.p[h], h, out.launches, batched, trace_blocks, false,
+                                      prof);
           out.launches += 1;
         }
       }
-      hipError_t e = hipStreamSynchronize(s);
+      // The sizes of the last iteration's queues, as its traversal starts: the
+      // next iteration is enqueued while it runs. (Profiling reads that
+      // traversal's events, so it waits for its end.)
+      const volatile gpu::WfReport *rep = r.wf_reports + h;
       if (out.err == hipSuccess)
-        out.err = e;
+        out.err = prof ? hipStreamSynchronize(s)
+                       : wait_report(rep, uint32_t(out.launches), s);
       if (out.err != hipSuccess) {
+        (void)hipStreamSynchronize(s); // nothing of this render is left running
         out.what = "launch / sync";
         break;
       }
-      // counts of the last iteration's queues (pinned host copy in the stream)
-      const uint32_t *c = r.wf_host_counts + size_t(h) * gpu::kNumCounters;
-      const uint32_t ne = c[gpu::kExtCount], ns = c[gpu::kShadowCount];
+      const uint32_t ne = rep->ext, ns = rep->shadow;
       if (prof && ne + ns) {
         float a = 0.f;
         (void)hipEventElapsedTime(&a, r.ev_prof[h][0], r.ev_prof[h][1]);
@@ -208,7 +263,24 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
       // a slot holds a path iff it queued at least one ray
       if (ne + ns == 0)
         break;
+      // Few paths are left and no sample is waiting for a slot: one launch
+      // takes them to their ends. A path has at most two queue entries.
+      if (!use_graph && !prof && rep->samples_left == 0 && ne + ns <= kFinishRays) {
+        const uint32_t entries = 2 * (ne + ns);
+        const uint32_t blocks =
+            std::min(trace_blocks, (entries + gpu::kFinishBlockPaths - 1) / gpu::kFinishBlockPaths);
+        out.err = enqueue_iteration(r, w.p[h], h, out.launches, batched, trace_blocks, false,
+                                    false, blocks);
+        out.launches += 1;
+        if (out.err != hipSuccess)
+          out.what = "launch";
+        break;
+      }
     }
+    // the last iteration's launches (they found empty queues) and the graph's
+    // last use
+    if (out.err == hipSuccess && (out.err = hipStreamSynchronize(s)) != hipSuccess)
+      out.what = "sync";
     if (exec)
       (void)hipGraphExecDestroy(exec);
   };

@@ -1,0 +1,68 @@
+"""The wavefront integrator's iterations and their end: both sets of queue
+counters, single-launch finishing of the last paths (from the first iteration
+for small images, after many regenerations with small pools), captured
+iterations. The mega-kernel, which has none of these, gives the image."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _settings(approach, term, rng):
+    from path_amd.renderer import Settings
+    s = Settings()
+    s.kernel_approach = approach
+    s.rng = rng
+    s.term_prob = term
+    s.n_iters = 5
+    s.constant_prob = 0.2
+    return s
+
+
+# 12 x 9 x 7: one ragged block, finished after one iteration; 128 x 96 x 1 and
+# 2: at and above the finishing limit; 301 x 97 x 30: three pipelines, finished
+# after several iterations; pool: fewer slots than samples
+@pytest.mark.parametrize("x,y,spp,pool,pipes", [
+    (1, 1, 1, 0, 0), (12, 9, 7, 0, 0), (128, 96, 1, 0, 0), (128, 96, 2, 0, 0),
+    (301, 97, 30, 0, 0), (64, 48, 9, 300, 1), (64, 48, 9, 5000, 4)])
+@pytest.mark.parametrize("which,term,rng", [
+    ("cornell", "Constant", "Uniform"), ("cornell_sphere", "Constant", "Sobel"),
+    ("cornell_sphere", "NIters", "Uniform")])
+def test_streaming_equals_megakernel(renderer, request, which, term, rng, x, y, spp, pool, pipes):
+    from path_amd.datagen import set_launch_params, set_pipelines
+    scene, ftw = request.getfixturevalue(which)
+    mega, _ = renderer.render(scene, ftw, x, y, spp, _settings("MegaKernel", term, rng))
+    rays = renderer.last_stats().rays
+    s = _settings("Streaming", term, rng)
+    if pool:
+        s.max_num_samples_per_launch = pool
+    try:
+        if pipes:
+            set_pipelines(renderer, pipes)
+        for iters, graphs in ((1, False), (3, False), (1, True), (3, True)):
+            set_launch_params(renderer, 0, iters, graphs)
+            img, _ = renderer.render(scene, ftw, x, y, spp, s)
+            assert np.array_equal(img.view(np.uint32), mega.view(np.uint32)), (iters, graphs)
+            assert renderer.last_stats().rays == rays, (iters, graphs)
+    finally:
+        set_launch_params(renderer, 0, 1, False)
+        if pipes:
+            set_pipelines(renderer, 3)
+
+
+# 1 and 3 samples: finished after the first iteration; 40: after several.
+@pytest.mark.parametrize("spp", [1, 3, 40])
+def test_batch_equals_single_renders(renderer, spp):
+    from path_amd.datagen import datagen_settings, generate_scene, render_batch
+    gens = [g for g in map(generate_scene, range(40)) if g.resolution <= 64][:3]
+    assert len({g.resolution for g in gens}) > 1
+    s = datagen_settings()
+    s.term_prob = "Constant"
+    s.constant_prob = 0.3
+    images, gbufs, _ = render_batch(renderer, gens, spp, s)
+    s.kernel_approach = "MegaKernel"
+    for g, img, gb in zip(gens, images, gbufs):
+        mega, _ = renderer.render(g.scene, g.film_to_world, g.resolution, g.resolution, spp, s)
+        assert np.array_equal(np.asarray(img).reshape(mega.shape).view(np.uint32),
+                              mega.view(np.uint32))
+        assert np.isfinite(gb).all() and np.abs(gb).sum() > 0
