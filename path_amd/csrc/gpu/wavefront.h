@@ -143,6 +143,16 @@ hipError_t launch_wf_finish(const WfParams &p, bool batched, uint32_t grid_block
 hipError_t launch_wf_reduce(const float *samples, const WorkDivision &wd,
                             uint32_t samples_per, float *out_rgb,
                             hipStream_t s);
+// The same for many images whose samples and pixels are concatenated, one
+// launch: each item has a work division of one sample block, all of block_size.
+struct WfReduceItem {
+  WorkDivision wd;
+  uint32_t block_begin; // first block of the item's total_num_blocks()
+  uint32_t pixel_off;
+};
+hipError_t launch_wf_reduce_batch(const float *samples, const WfReduceItem *items, uint32_t n,
+                                  uint32_t block_size, uint32_t total_blocks,
+                                  uint32_t samples_per, float *out_rgb, hipStream_t s);
 // out[pixel] = (sum over the pixel's samples, sequential in FP64) / spp
 hipError_t launch_sum_samples_f64(const float *samples, uint32_t n_pixels,
                                   uint32_t samples_per, double *out, hipStream_t s);

@@ -552,32 +552,51 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
   if (rc != PT_OK)
     return rc;
   HIP_TRY(r.rgb.ensure(size_t(n_pixels) * 3));
+  std::vector<gpu::WfReduceItem> reduce, split_reduce;
+  uint32_t reduce_blocks = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    gpu::WfReduceItem it{};
+    if (!WorkDivision::make(work_division_settings(settings.render_work_division), spp,
+                            items[i].x_dim, items[i].y_dim, &it.wd) ||
+        it.wd.block_size > 1024)
+      return set_error(PT_ERR_INVALID, "invalid render work division settings");
+    it.pixel_off = desc[i].pixel_off;
+    it.block_begin = reduce_blocks;
+    const uint64_t blocks = uint64_t(reduce_blocks) + it.wd.total_num_blocks();
+    // (a grid of at most 2^32 - 1 threads)
+    if (it.wd.num_sample_blocks == 1 && blocks * it.wd.block_size <= 0xffffffffull) {
+      reduce.push_back(it);
+      reduce_blocks = uint32_t(blocks);
+    } else {
+      split_reduce.push_back(it);
+    }
+  }
+  HIP_TRY(r.b_reduce.upload(reduce.data(), reduce.size(), s));
   r.stats = pt_render_stats{};
   r.stats.profiled = r.profiling ? 1u : 0u;
   HIP_TRY(hipEventRecord(r.ev_start, s));
   rc = wavefront_run(r, w, true, trace_blocks, r.iters_per_sync);
   if (rc != PT_OK)
     return rc;
-  // per-scene reduction in the single-scene order
-  for (uint32_t i = 0; i < n; ++i) {
-    const pt_batch_item &it = items[i];
-    WorkDivision wd;
-    if (!WorkDivision::make(work_division_settings(settings.render_work_division), spp,
-                            it.x_dim, it.y_dim, &wd) ||
-        wd.block_size > 1024)
-      return set_error(PT_ERR_INVALID, "invalid render work division settings");
-    size_t off = desc[i].pixel_off;
-    size_t px = size_t(it.x_dim) * it.y_dim;
-    if (wd.num_sample_blocks == 1) {
-      HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, wd, spp,
+  // the reductions in the single-scene order: one launch
+  if (!reduce.empty()) {
+    HIP_TRY(gpu::launch_wf_reduce_batch(r.wf_samples.ptr, r.b_reduce.ptr, uint32_t(reduce.size()),
+                                        reduce[0].wd.block_size, reduce_blocks, spp, r.rgb.ptr,
+                                        s));
+  }
+  // and one or two each for scenes whose pixels have several sample blocks
+  // (or that did not fit the grid)
+  for (const gpu::WfReduceItem &it : split_reduce) {
+    const size_t off = it.pixel_off, px = size_t(it.wd.x_dim) * it.wd.y_dim;
+    if (it.wd.num_sample_blocks == 1) {
+      HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, it.wd, spp,
                                     r.rgb.ptr + 3 * off, s));
-    } else {
-      HIP_TRY(r.rgb2.ensure(px * 3 * wd.num_sample_blocks));
-      HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, wd, spp,
-                                    r.rgb2.ptr, s));
-      HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, wd.num_sample_blocks,
-                                               uint32_t(px), spp, r.rgb.ptr + 3 * off, s));
+      continue;
     }
+    HIP_TRY(r.rgb2.ensure(px * 3 * it.wd.num_sample_blocks));
+    HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, it.wd, spp, r.rgb2.ptr, s));
+    HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, it.wd.num_sample_blocks, uint32_t(px),
+                                             spp, r.rgb.ptr + 3 * off, s));
   }
   HIP_TRY(hipEventRecord(r.ev_stop, s));
   const size_t rgb_bytes = size_t(n_pixels) * 3 * sizeof(float);

@@ -223,6 +223,7 @@ struct pt_renderer {
   pt::host::DeviceBuf<float> b_light_cdf;
   pt::host::DeviceBuf<pt::gpu::SceneDesc> b_desc;
   pt::host::DeviceBuf<unsigned long long> b_sample_begin;
+  pt::host::DeviceBuf<pt::gpu::WfReduceItem> b_reduce;
   pt::host::DeviceBuf<float> b_gbuffer;
   pt::host::PinnedBuf b_stage_in, b_stage_out;
   pt::host::PinnedBuf out_stage; // host outputs of pt_render

@@ -51,14 +51,19 @@ def test_streaming_equals_megakernel(renderer, request, which, term, rng, x, y, 
 
 
 # 1 and 3 samples: finished after the first iteration; 40: after several.
-@pytest.mark.parametrize("spp", [1, 3, 40])
-def test_batch_equals_single_renders(renderer, spp):
+# forced 1 sample per thread and 512 samples: several sample blocks per pixel
+# (two reduction passes); the others are reduced in one launch
+@pytest.mark.parametrize("spp,forced", [(1, 0), (3, 0), (40, 0), (512, 1)])
+def test_batch_equals_single_renders(renderer, spp, forced):
     from path_amd.datagen import datagen_settings, generate_scene, render_batch
     gens = [g for g in map(generate_scene, range(40)) if g.resolution <= 64][:3]
     assert len({g.resolution for g in gens}) > 1
     s = datagen_settings()
     s.term_prob = "Constant"
     s.constant_prob = 0.3
+    if forced:
+        s.render_work_division.force_target_samples = 1
+        s.render_work_division.forced_target_samples_per_thread = forced
     images, gbufs, _ = render_batch(renderer, gens, spp, s)
     s.kernel_approach = "MegaKernel"
     for g, img, gb in zip(gens, images, gbufs):
