@@ -417,7 +417,7 @@ constexpr uint32_t kRefillMinIdle = 16;
 // 2 / 3 / 4 / 5 / 6: 881-883 / 895-898 / 902-903 / 899-900 / 898-899 (the
 // batched scenes: no difference between 3 and 4); refill thresholds 8 / 16 /
 // 24 / 32: 884 / 895-898 / 899-900 / 887.
-constexpr uint32_t kTraceVote = 4;
+constexpr int kTraceVote = 4;
 // Wave 0 of a block: s_prefix[g] = first entry of segment g of the
 // concatenated queues (extension segments, then shadow segments). Returns the
 // lane's inclusive sum.
@@ -515,14 +515,15 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
   TraceState ts;
   const float4 *nodes = p.scene.nodes, *tris = p.scene.tris;
   uint32_t slot = 0;
-  bool has = false, shadow = false;
+  bool shadow = false;
+  ts.node = TraceState::kNoRef;
   for (;;) {
-    const uint64_t idle = __ballot(!has);
-    const uint32_t n_idle = uint32_t(__popcll(idle));
+    const uint64_t idle = ballot(ts.idle());
+    const uint32_t n_idle = uint32_t(count_lanes(idle));
     if (next < end && (n_idle >= kRefillMinIdle || n_idle == 64u)) {
       const uint32_t pre = __builtin_amdgcn_mbcnt_hi(
           uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
-      if (!has && next + pre < end) {
+      if (ts.idle() && next + pre < end) {
         const uint32_t j = next + pre;
         const uint32_t v = j < e_len ? e0 + j : n_ext + s0 + (j - e_len);
         slot = queue_slot(p, s_prefix, v, &shadow);
@@ -544,22 +545,20 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
         }
         ts.init(ray, shadow ? d.w + 2e-6f : 3.4028235e38f, shadow ? d.w - 2e-6f : -1.0f);
         stack.sp = 0;
-        if (has_nodes && ray_can_hit(ray))
-          has = true;
-        else
+        if (!has_nodes || !ray_can_hit(ray)) {
+          ts.node = TraceState::kNoRef;
           (shadow ? p.st.hit_light : p.st.hit_ext)[slot] = pack_hit(Hit<float>{0.f, kNoHit, 0});
+        }
       }
       next = min(next + n_idle, end);
     }
-    if (__ballot(has) == 0) {
+    if (ballot(!ts.idle()) == 0) {
       if (next >= end)
         break;
       continue;
     }
-    if (ts.step_voted(nodes, tris, stack, has, kTraceVote)) {
+    if (ts.step_voted(nodes, tris, stack, kTraceVote))
       (shadow ? p.st.hit_light : p.st.hit_ext)[slot] = pack_hit(ts.hit());
-      has = false;
-    }
   }
 }
 
