@@ -86,6 +86,13 @@ struct SceneDesc {
   float film_to_world[12];
 };
 
+// What a wavefront render's samples are.
+enum WfKind : int {
+  kWfImage, // pixels of one scene's image
+  kWfBatch, // pixels of many scenes' images (WfBatch)
+  kWfRays,  // given rays of many scenes (WfBatch: scene i has x_dim rays)
+};
+
 struct WfBatch {
   const SceneDesc *scenes;
   const unsigned long long *sample_begin; // n_scenes + 1 prefix of pixels*spp
@@ -95,6 +102,11 @@ struct WfBatch {
   const Material<float> *materials;
   const TriGeom<float> *light_tris;
   const float *light_cdf;
+  // kWfRays: 6 floats per ray; triangle each ray hits first at distance 1
+  // (InitialIdxAndDir), or null; per-step outputs (0: one value per sample)
+  const float *rays;
+  const uint32_t *initial_idx;
+  uint32_t n_steps;
 };
 
 struct WfParams {
@@ -119,24 +131,26 @@ struct WfParams {
   // path pool can be split into independent pipelines on separate streams):
   // this launch's group g is group group_base + g of n_groups_total.
   uint32_t group_base, n_groups_total;
-  float *out_samples;                 // [pixel * spp + sample] * 3
+  // [pixel * spp + sample] * 3; with n_steps one such array per step, zero
+  // where a path ends before the step
+  float *out_samples;
   float *gbuffer; // first hit of sample 0 per pixel: position, normal,
                   // albedo, emission (12 floats) or null
   int *stack_overflow;                // traversal stack spill area
   uint32_t overflow_stride;           // threads of a traversal launch
 };
 
-hipError_t launch_wf_shade(const WfParams &p, bool batched, hipStream_t s);
+hipError_t launch_wf_shade(const WfParams &p, WfKind kind, hipStream_t s);
 // Closest hits of the iteration's extension rays and occlusion of its shadow
 // rays, both queues in one launch; also adds the iteration's queue counts to
 // the totals, reports them to the host and zeroes the other set of counters.
-hipError_t launch_wf_trace(const WfParams &p, bool batched, uint32_t grid_blocks,
+hipError_t launch_wf_trace(const WfParams &p, WfKind kind, uint32_t grid_blocks,
                            hipStream_t s);
 // Takes the paths of the iteration's queues to their ends, each lane tracing
 // its own rays, instead of launch_wf_trace: for an iteration after which few
 // paths and no samples are left.
 constexpr uint32_t kFinishBlockPaths = 64; // queue entries per block and round
-hipError_t launch_wf_finish(const WfParams &p, bool batched, uint32_t grid_blocks,
+hipError_t launch_wf_finish(const WfParams &p, WfKind kind, uint32_t grid_blocks,
                             hipStream_t s);
 // Per-pixel sum of the per-sample radiance in the mega-kernel's order
 // (sequential per thread range, then the lane tree), divided by spp.

@@ -184,8 +184,22 @@ __device__ __forceinline__ void write_sample(const WfParams &p, const SlotScene 
   out[2] = radiance.z;
 }
 
-template <class R, bool kBatch>
+// Radiance the iteration after `iters` iterations of a kWfRays path added.
+__device__ __forceinline__ void write_step(const WfParams &p, const SlotScene &sc,
+                                           uint32_t location, uint32_t sample, uint32_t iters,
+                                           V3<float> added) {
+  const size_t i = size_t(iters) * p.total_samples +
+                   size_t(sc.pixel_off + location) * p.rng.samples_per + sample;
+  p.out_samples[3 * i] = added.x;
+  p.out_samples[3 * i + 1] = added.y;
+  p.out_samples[3 * i + 2] = added.z;
+}
+
+template <class R, int kKind>
 __device__ __forceinline__ void wf_shade(const WfParams &p) {
+  constexpr bool kBatch = kKind != kWfImage;
+  // each iteration's radiance is an output of its own
+  const bool steps = kKind == kWfRays && p.batch.n_steps != 0;
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t group = blockIdx.x % p.n_groups;
   const bool in_range = slot < p.n_slots;
@@ -208,7 +222,9 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
   if (active) {
     SlotScene sc = slot_scene<kBatch>(p, scene);
     Ray<float> last;
-    const PathState<float> st = load_path(p, slot, meta.w, &last);
+    PathState<float> st = load_path(p, slot, meta.w, &last);
+    if (steps)
+      st.total = {0.f, 0.f, 0.f};
     Hit<float> light_hit = {0.f, kNoHit, 0}, next_hit = {0.f, kNoHit, 0};
     if (st.n_light)
       light_hit = unpack_hit(p.st.hit_light[slot]);
@@ -229,8 +245,13 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
     counter = rng_counter(rng);
     total_dirty =
         ns.total.x != st.total.x || ns.total.y != st.total.y || ns.total.z != st.total.z;
+    if (steps) {
+      write_step(p, sc, location, sample, st.iters, ns.total);
+      finished = finished || ns.iters >= p.batch.n_steps;
+    }
     if (finished) {
-      write_sample(p, sc, location, sample, ns.total);
+      if (!steps)
+        write_sample(p, sc, location, sample, ns.total);
     } else {
       if (ns.n_light) {
         push_light = true;
@@ -285,11 +306,16 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
       location = uint32_t(local / p.rng.samples_per);
       sample = uint32_t(local % p.rng.samples_per);
       R rng = make_rng<R>(p.rng, location, sample, rng_start<R>(p.rng, location));
-      float xo = rng.next();
-      float yo = rng.next();
-      uint32_t px = location % sc.x_dim, py = location / sc.x_dim;
-      Ray<float> cam = camera_ray(sc.film_to_world, float(px) + xo,
-                                  float(py) + yo, sc.x_dim, sc.y_dim);
+      Ray<float> cam;
+      if constexpr (kKind == kWfRays) {
+        const float *r = p.batch.rays + 6 * size_t(sc.pixel_off + location);
+        cam = {{r[0], r[1], r[2]}, {r[3], r[4], r[5]}};
+      } else {
+        float xo = rng.next();
+        float yo = rng.next();
+        uint32_t px = location % sc.x_dim, py = location / sc.x_dim;
+        cam = camera_ray(sc.film_to_world, float(px) + xo, float(py) + yo, sc.x_dim, sc.y_dim);
+      }
       counter = rng_counter(rng);
       ns = initial_path_state<float>();
       total_dirty = true;
@@ -360,30 +386,39 @@ __device__ __forceinline__ void wf_shade(const WfParams &p) {
 // 7 waves measured 133.5). A single render asks for at least 6, which the
 // compiler's own allocation (68 VGPRs, 7 waves, no spills) already meets;
 // asking 8 there spilled more and measured slower.
-template <class R, bool kBatch>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatch ? 8 : 6))) void
+template <class R, int kKind>
+__global__
+__launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kKind != kWfImage ? 8 : 6))) void
 k_wf_shade(WfParams p) {
-  wf_shade<R, kBatch>(p);
+  wf_shade<R, kKind>(p);
 }
 
-hipError_t launch_wf_shade(const WfParams &p, bool batched, hipStream_t s) {
+// f<R, kind>() for the render's generator and kind.
+template <class F> static void dispatch_wf(const WfParams &p, WfKind kind, F f) {
+  auto with = [&](auto r) {
+    using R = decltype(r);
+    if (kind == kWfImage)
+      f.template operator()<R, kWfImage>();
+    else if (kind == kWfBatch)
+      f.template operator()<R, kWfBatch>();
+    else
+      f.template operator()<R, kWfRays>();
+  };
+  if (p.rng.type == kRngSobel)
+    with(TableRng{});
+  else
+    with(HashRng{});
+}
+
+hipError_t launch_wf_shade(const WfParams &p, WfKind kind, hipStream_t s) {
   uint32_t blocks = (p.n_slots + 255) / 256;
   // groups and sample shares are laid out for exactly this grid
   if (blocks != p.n_shade_blocks || p.n_groups == 0 || p.n_groups > kQueueGroups ||
       p.n_groups > blocks || p.group_base + p.n_groups > p.n_groups_total)
     return hipErrorInvalidValue;
-  bool sobol = p.rng.type == kRngSobel;
-  if (batched) {
-    if (sobol)
-      hipLaunchKernelGGL((k_wf_shade<TableRng, true>), dim3(blocks), dim3(256), 0, s, p);
-    else
-      hipLaunchKernelGGL((k_wf_shade<HashRng, true>), dim3(blocks), dim3(256), 0, s, p);
-  } else {
-    if (sobol)
-      hipLaunchKernelGGL((k_wf_shade<TableRng, false>), dim3(blocks), dim3(256), 0, s, p);
-    else
-      hipLaunchKernelGGL((k_wf_shade<HashRng, false>), dim3(blocks), dim3(256), 0, s, p);
-  }
+  dispatch_wf(p, kind, [&]<class R, int kKind>() {
+    hipLaunchKernelGGL((k_wf_shade<R, kKind>), dim3(blocks), dim3(256), 0, s, p);
+  });
   return hipGetLastError();
 }
 
@@ -418,6 +453,16 @@ constexpr uint32_t kRefillMinIdle = 16;
 // batched scenes: no difference between 3 and 4); refill thresholds 8 / 16 /
 // 24 / 32: 884 / 895-898 / 899-900 / 887.
 constexpr int kTraceVote = 4;
+// The hit a kWfRays path starts with, if it is given (InitialIdxAndDir: at
+// distance 1 and front-facing by convention, initial_ray_sample.h:58-75).
+__device__ __forceinline__ bool given_hit(const WfParams &p, uint4 meta, uint32_t scene,
+                                          Hit<float> *hit) {
+  if (!p.batch.initial_idx || (meta.w & kItersMask) != 0)
+    return false;
+  *hit = {1.f, p.batch.initial_idx[size_t(p.batch.scenes[scene].pixel_off) + meta.x], 0};
+  return true;
+}
+
 // Wave 0 of a block: s_prefix[g] = first entry of segment g of the
 // concatenated queues (extension segments, then shadow segments). Returns the
 // lane's inclusive sum.
@@ -457,8 +502,8 @@ __device__ __forceinline__ uint32_t queue_slot(const WfParams &p, const uint32_t
 // launch measured 757 -> 856 Msamples/s on the 82k-triangle scene (C3 fresh
 // scenes 4,671 -> 5,056 scenes/s): one tail per iteration instead of two, and
 // waves that finish their extension rays continue with shadow rays.
-template <bool kBatch>
-__device__ __forceinline__ void wf_trace(const WfParams &p) {
+template <int kKind> __device__ __forceinline__ void wf_trace(const WfParams &p) {
+  constexpr bool kBatch = kKind != kWfImage;
   __shared__ int lds_stack[kLdsStackInts * 4];
   __shared__ uint32_t s_prefix[2 * kQueueGroups + 1];
   if (threadIdx.x < 64) {
@@ -549,6 +594,13 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
           ts.node = TraceState::kNoRef;
           (shadow ? p.st.hit_light : p.st.hit_ext)[slot] = pack_hit(Hit<float>{0.f, kNoHit, 0});
         }
+        if constexpr (kKind == kWfRays) {
+          Hit<float> given;
+          if (!shadow && given_hit(p, p.st.meta[slot], p.st.scene[slot], &given)) {
+            ts.node = TraceState::kNoRef;
+            p.st.hit_ext[slot] = pack_hit(given);
+          }
+        }
       }
       next = min(next + n_idle, end);
     }
@@ -566,18 +618,22 @@ __device__ __forceinline__ void wf_trace(const WfParams &p) {
 // of many small scenes (1024 generated scenes: render 133.9 -> 132.1 ms, no
 // spills), the compiler's 7 (67 VGPRs) for a single render (with 8 the
 // 82k-triangle scene measured 874 vs 899 Msamples/s).
-template <bool kBatch>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatch ? 8 : 7))) void
+template <int kKind>
+__global__
+__launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kKind != kWfImage ? 8 : 7))) void
 k_wf_trace(WfParams p) {
-  wf_trace<kBatch>(p);
+  wf_trace<kKind>(p);
 }
 
-hipError_t launch_wf_trace(const WfParams &p, bool batched, uint32_t grid_blocks,
+hipError_t launch_wf_trace(const WfParams &p, WfKind kind, uint32_t grid_blocks,
                            hipStream_t s) {
-  if (batched)
-    hipLaunchKernelGGL((k_wf_trace<true>), dim3(grid_blocks), dim3(256), 0, s, p);
+  const dim3 grid(grid_blocks), block(256);
+  if (kind == kWfImage)
+    hipLaunchKernelGGL(k_wf_trace<kWfImage>, grid, block, 0, s, p);
+  else if (kind == kWfBatch)
+    hipLaunchKernelGGL(k_wf_trace<kWfBatch>, grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL((k_wf_trace<false>), dim3(grid_blocks), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(k_wf_trace<kWfRays>, grid, block, 0, s, p);
   return hipGetLastError();
 }
 
@@ -589,8 +645,10 @@ hipError_t launch_wf_trace(const WfParams &p, bool batched, uint32_t grid_blocks
 // so the results are the same bits.
 constexpr uint32_t kFinishLanes = kFinishBlockPaths / 4;
 
-template <class R, bool kBatch>
+template <class R, int kKind>
 __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
+  constexpr bool kBatch = kKind != kWfImage;
+  const bool steps = kKind == kWfRays && p.batch.n_steps != 0;
   __shared__ int lds_stack[kLdsStackInts * 4];
   __shared__ uint32_t s_prefix[2 * kQueueGroups + 1];
   if (threadIdx.x < 64)
@@ -627,7 +685,13 @@ __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
       light_ray.d = {d.x, d.y, d.z};
     }
     R rng = make_rng<R>(p.rng, location, sample, meta.z);
+    Hit<float> given = {0.f, kNoHit, 0};
+    bool is_given = false;
+    if constexpr (kKind == kWfRays)
+      is_given = given_hit(p, meta, scene, &given);
     for (;;) {
+      if (steps)
+        st.total = {0.f, 0.f, 0.f};
       Hit<float> light_hit = {0.f, kNoHit, 0}, next_hit = {0.f, kNoHit, 0};
       if (st.n_light) {
         ++n_shadow;
@@ -637,19 +701,27 @@ __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
       }
       if (st.has_next) {
         ++n_ext;
-        if (has_nodes)
+        if (is_given)
+          next_hit = given;
+        else if (has_nodes)
           next_hit = trace_closest(nodes, tris, last, 3.4028235e38f, -1.0f, stack);
       }
       PathState<float> ns;
       Ray<float> nl = light_ray, nn = last;
       VertexInfo<float> vi;
       vi.valid = 0u;
-      const bool done = rendering_equation_iteration(st, rng, last, light_hit, next_hit,
-                                                     p.settings, sc.view, &ns, &nl, &nn, &vi);
+      bool done = rendering_equation_iteration(st, rng, last, light_hit, next_hit, p.settings,
+                                               sc.view, &ns, &nl, &nn, &vi);
+      is_given = false;
+      if (steps) {
+        write_step(p, sc, location, sample, st.iters, ns.total);
+        done = done || ns.iters >= p.batch.n_steps;
+      }
       if (p.gbuffer && st.iters == 0 && sample == 0 && vi.valid)
         write_gbuffer(p, sc, location, vi);
       if (done) {
-        write_sample(p, sc, location, sample, ns.total);
+        if (!steps)
+          write_sample(p, sc, location, sample, ns.total);
         break;
       }
       st = ns;
@@ -670,20 +742,13 @@ __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
   }
 }
 
-hipError_t launch_wf_finish(const WfParams &p, bool batched, uint32_t grid_blocks,
+hipError_t launch_wf_finish(const WfParams &p, WfKind kind, uint32_t grid_blocks,
                             hipStream_t s) {
   if (grid_blocks == 0 || uint64_t(grid_blocks) * 256 > p.overflow_stride)
     return hipErrorInvalidValue;
-  const dim3 grid(grid_blocks), block(256);
-  const bool sobol = p.rng.type == kRngSobel;
-  if (batched && sobol)
-    hipLaunchKernelGGL((k_wf_finish<TableRng, true>), grid, block, 0, s, p);
-  else if (batched)
-    hipLaunchKernelGGL((k_wf_finish<HashRng, true>), grid, block, 0, s, p);
-  else if (sobol)
-    hipLaunchKernelGGL((k_wf_finish<TableRng, false>), grid, block, 0, s, p);
-  else
-    hipLaunchKernelGGL((k_wf_finish<HashRng, false>), grid, block, 0, s, p);
+  dispatch_wf(p, kind, [&]<class R, int kKind>() {
+    hipLaunchKernelGGL((k_wf_finish<R, kKind>), dim3(grid_blocks), dim3(256), 0, s, p);
+  });
   return hipGetLastError();
 }
 

@@ -460,6 +460,62 @@ int ensure_batch_scenes(pt_renderer &r, const pt_batch_item *items, uint32_t n, 
   return PT_OK;
 }
 
+// The wavefront's view of the batch arrays of n scenes.
+gpu::WfBatch wavefront_batch(const pt_renderer &r, uint32_t n) {
+  gpu::WfBatch b{};
+  b.scenes = r.b_desc.ptr;
+  b.sample_begin = r.b_sample_begin.ptr;
+  b.n_scenes = n;
+  b.nodes = reinterpret_cast<const float4 *>(r.b_nodes.ptr);
+  b.tris = reinterpret_cast<const float4 *>(r.b_tris.ptr);
+  b.shade = r.b_shade.ptr;
+  b.materials = r.b_mats.ptr;
+  b.light_tris = r.b_light_tris.ptr;
+  b.light_cdf = r.b_light_cdf.ptr;
+  return b;
+}
+
+// Per-pixel sums of a batch's images, each in its single-render order: one
+// launch for all images whose pixels have one sample block; the others (and
+// images that no longer fit the grid) in launches of their own.
+struct BatchReduction {
+  std::vector<gpu::WfReduceItem> together, alone;
+  uint32_t blocks = 0;
+
+  void add(const WorkDivision &wd, uint32_t pixel_off) {
+    const uint64_t end = uint64_t(blocks) + wd.total_num_blocks();
+    // (a grid of at most 2^32 - 1 threads)
+    if (wd.num_sample_blocks == 1 && end * wd.block_size <= 0xffffffffull) {
+      together.push_back({wd, blocks, pixel_off});
+      blocks = uint32_t(end);
+    } else {
+      alone.push_back({wd, 0, pixel_off});
+    }
+  }
+  int upload(pt_renderer &r) const {
+    HIP_TRY(r.b_reduce.upload(together.data(), together.size(), r.stream));
+    return PT_OK;
+  }
+  int run(pt_renderer &r, const float *samples, uint32_t spp, float *out) const {
+    hipStream_t s = r.stream;
+    if (!together.empty())
+      HIP_TRY(gpu::launch_wf_reduce_batch(samples, r.b_reduce.ptr, uint32_t(together.size()),
+                                          together[0].wd.block_size, blocks, spp, out, s));
+    for (const gpu::WfReduceItem &it : alone) {
+      const size_t off = it.pixel_off, px = size_t(it.wd.x_dim) * it.wd.y_dim;
+      if (it.wd.num_sample_blocks == 1) {
+        HIP_TRY(gpu::launch_wf_reduce(samples + 3 * off * spp, it.wd, spp, out + 3 * off, s));
+        continue;
+      }
+      HIP_TRY(r.rgb2.ensure(px * 3 * it.wd.num_sample_blocks));
+      HIP_TRY(gpu::launch_wf_reduce(samples + 3 * off * spp, it.wd, spp, r.rgb2.ptr, s));
+      HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, it.wd.num_sample_blocks, uint32_t(px),
+                                               spp, out + 3 * off, s));
+    }
+    return PT_OK;
+  }
+};
+
 } // namespace
 
 namespace pt {
@@ -530,15 +586,7 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
   gpu::WfParams p{};
   p.settings = integrator_settings(settings);
   p.rng = rng;
-  p.batch.scenes = r.b_desc.ptr;
-  p.batch.sample_begin = r.b_sample_begin.ptr;
-  p.batch.n_scenes = n;
-  p.batch.nodes = reinterpret_cast<const float4 *>(r.b_nodes.ptr);
-  p.batch.tris = reinterpret_cast<const float4 *>(r.b_tris.ptr);
-  p.batch.shade = r.b_shade.ptr;
-  p.batch.materials = r.b_mats.ptr;
-  p.batch.light_tris = r.b_light_tris.ptr;
-  p.batch.light_cdf = r.b_light_cdf.ptr;
+  p.batch = wavefront_batch(r, n);
   bool want_gbuffer = false;
   for (uint32_t i = 0; i < n; ++i)
     want_gbuffer |= items[i].out_gbuffer != nullptr;
@@ -548,56 +596,30 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
     p.gbuffer = r.b_gbuffer.ptr;
   }
   WfPipes w;
-  rc = wavefront_alloc(r, w, p, uint32_t(slots), total, true, trace_blocks);
+  rc = wavefront_alloc(r, w, p, uint32_t(slots), total, gpu::kWfBatch, trace_blocks);
   if (rc != PT_OK)
     return rc;
   HIP_TRY(r.rgb.ensure(size_t(n_pixels) * 3));
-  std::vector<gpu::WfReduceItem> reduce, split_reduce;
-  uint32_t reduce_blocks = 0;
+  BatchReduction red;
   for (uint32_t i = 0; i < n; ++i) {
-    gpu::WfReduceItem it{};
+    WorkDivision wd;
     if (!WorkDivision::make(work_division_settings(settings.render_work_division), spp,
-                            items[i].x_dim, items[i].y_dim, &it.wd) ||
-        it.wd.block_size > 1024)
+                            items[i].x_dim, items[i].y_dim, &wd) ||
+        wd.block_size > 1024)
       return set_error(PT_ERR_INVALID, "invalid render work division settings");
-    it.pixel_off = desc[i].pixel_off;
-    it.block_begin = reduce_blocks;
-    const uint64_t blocks = uint64_t(reduce_blocks) + it.wd.total_num_blocks();
-    // (a grid of at most 2^32 - 1 threads)
-    if (it.wd.num_sample_blocks == 1 && blocks * it.wd.block_size <= 0xffffffffull) {
-      reduce.push_back(it);
-      reduce_blocks = uint32_t(blocks);
-    } else {
-      split_reduce.push_back(it);
-    }
+    red.add(wd, desc[i].pixel_off);
   }
-  HIP_TRY(r.b_reduce.upload(reduce.data(), reduce.size(), s));
+  if ((rc = red.upload(r)) != PT_OK)
+    return rc;
   r.stats = pt_render_stats{};
   r.stats.profiled = r.profiling ? 1u : 0u;
   HIP_TRY(hipEventRecord(r.ev_start, s));
-  rc = wavefront_run(r, w, true, trace_blocks, r.iters_per_sync);
+  rc = wavefront_run(r, w, gpu::kWfBatch, trace_blocks, r.iters_per_sync);
   if (rc != PT_OK)
     return rc;
-  // the reductions in the single-scene order: one launch
-  if (!reduce.empty()) {
-    HIP_TRY(gpu::launch_wf_reduce_batch(r.wf_samples.ptr, r.b_reduce.ptr, uint32_t(reduce.size()),
-                                        reduce[0].wd.block_size, reduce_blocks, spp, r.rgb.ptr,
-                                        s));
-  }
-  // and one or two each for scenes whose pixels have several sample blocks
-  // (or that did not fit the grid)
-  for (const gpu::WfReduceItem &it : split_reduce) {
-    const size_t off = it.pixel_off, px = size_t(it.wd.x_dim) * it.wd.y_dim;
-    if (it.wd.num_sample_blocks == 1) {
-      HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, it.wd, spp,
-                                    r.rgb.ptr + 3 * off, s));
-      continue;
-    }
-    HIP_TRY(r.rgb2.ensure(px * 3 * it.wd.num_sample_blocks));
-    HIP_TRY(gpu::launch_wf_reduce(r.wf_samples.ptr + 3 * off * spp, it.wd, spp, r.rgb2.ptr, s));
-    HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, it.wd.num_sample_blocks, uint32_t(px),
-                                             spp, r.rgb.ptr + 3 * off, s));
-  }
+  // the reductions in the single-scene order
+  if ((rc = red.run(r, r.wf_samples.ptr, spp, r.rgb.ptr)) != PT_OK)
+    return rc;
   HIP_TRY(hipEventRecord(r.ev_stop, s));
   const size_t rgb_bytes = size_t(n_pixels) * 3 * sizeof(float);
   const size_t gb_bytes = want_gbuffer ? size_t(n_pixels) * 12 * sizeof(float) : 0;
@@ -649,6 +671,91 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
   r.stats.kernel_ms = ms;
   r.stats.samples = total;
   r.stats.rays = r.stats.ext_rays + r.stats.shadow_rays;
+  if (seconds)
+    *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  return PT_OK;
+}
+
+// The wavefront traces a batch's rays from this many samples on, and of three
+// steps or more: the mega-kernel's waves wait for their longest path, the
+// wavefront pays two launches an iteration. Whole calls, us, mega-kernel /
+// wavefront, six steps: 89,600 samples 1,102 / 1,015, 192,000: 1,292 / 1,356,
+// 384,000: 1,684 / 1,321, 1.15 M: 3,387 / 2,479; no steps: 240,000: 1,449 /
+// 1,237, 768,000: 2,305 / 1,834; three steps, 576,000: 1,323 / 1,051; one step,
+// 192,000: 579 / 637, 1.15 M: 907 / 952. Its per-sample values may take this
+// many bytes.
+constexpr uint64_t kRaysWavefrontMin = 1u << 18;
+constexpr size_t kRaysWavefrontBytes = size_t(4) << 30;
+
+// The wavefront's part of render_rays_batch: scenes, rays and indices are on the
+// device. Values are summed like the mega-kernel's, so they are the same bits.
+// *no_memory is set, and nothing done, if its buffers do not fit the device.
+static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
+                          const std::vector<uint32_t> &act,
+                          const std::vector<gpu::SceneDesc> &desc,
+                          const std::vector<gpu::MegaBatchItem> &mb, const pt_settings &settings,
+                          const gpu::RngParams &rng, bool with_idx, uint32_t n_steps,
+                          uint64_t total, uint64_t n_rays,
+                          std::chrono::steady_clock::time_point t0, double *seconds,
+                          bool *no_memory) {
+  hipStream_t s = r.stream;
+  const uint32_t n_img = n_steps ? n_steps : 1, m = uint32_t(act.size());
+  if (r.ray_samples.ensure(size_t(n_img) * total * 3) != hipSuccess) {
+    (void)hipGetLastError();
+    *no_memory = true;
+    return PT_OK;
+  }
+  HIP_TRY(r.rgb.ensure(size_t(n_img) * n_rays * 3));
+  gpu::WfParams p{};
+  p.settings = integrator_settings(settings);
+  p.rng = rng;
+  p.batch = wavefront_batch(r, m);
+  p.batch.rays = r.scratch_rays.ptr;
+  p.batch.initial_idx = with_idx ? r.scratch_idx.ptr : nullptr;
+  p.batch.n_steps = n_steps;
+  p.out_samples = r.ray_samples.ptr;
+  // (max_num_samples_per_launch is the Streaming integrator's setting)
+  const uint64_t slots = std::min<uint64_t>(1u << 22, total);
+  const uint32_t trace_blocks = uint32_t(r.n_cus) * r.trace_blocks_for(true);
+  WfPipes w;
+  int rc = wavefront_alloc(r, w, p, uint32_t(slots), total, gpu::kWfRays, trace_blocks);
+  if (rc != PT_OK) {
+    (void)hipGetLastError();
+    *no_memory = true;
+    return PT_OK;
+  }
+  BatchReduction red;
+  for (uint32_t j = 0; j < m; ++j)
+    red.add(mb[j].wd, desc[j].pixel_off);
+  if ((rc = red.upload(r)) != PT_OK)
+    return rc;
+  HIP_TRY(hipEventRecord(r.ev_start, s));
+  if (n_steps) // steps that a path does not reach stay zero
+    HIP_TRY(hipMemsetAsync(r.ray_samples.ptr, 0, size_t(n_img) * total * 3 * sizeof(float), s));
+  if ((rc = wavefront_run(r, w, gpu::kWfRays, trace_blocks, r.iters_per_sync)) != PT_OK)
+    return rc;
+  for (uint32_t k = 0; k < n_img; ++k)
+    if ((rc = red.run(r, r.ray_samples.ptr + size_t(k) * total * 3, rng.samples_per,
+                      r.rgb.ptr + size_t(k) * n_rays * 3)) != PT_OK)
+      return rc;
+  HIP_TRY(hipEventRecord(r.ev_stop, s));
+  const size_t bytes = size_t(n_img) * n_rays * 3 * sizeof(float);
+  HIP_TRY(r.b_stage_out.ensure(bytes));
+  const float *out = static_cast<const float *>(r.b_stage_out.ptr);
+  HIP_TRY(hipMemcpyAsync(r.b_stage_out.ptr, r.rgb.ptr, bytes, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  for (uint32_t j = 0; j < m; ++j) {
+    const size_t nr = items[act[j]].n_rays;
+    for (uint32_t k = 0; k < n_img; ++k)
+      std::memcpy(items[act[j]].out + size_t(k) * nr * 3,
+                  out + (size_t(k) * n_rays + desc[j].pixel_off) * 3, nr * 3 * sizeof(float));
+  }
+  float ms = 0.f;
+  HIP_TRY(hipEventElapsedTime(&ms, r.ev_start, r.ev_stop));
+  r.stats.kernel_ms = ms;
+  // given first hits went through the queues untraced
+  r.stats.rays = r.stats.ext_rays + r.stats.shadow_rays - (with_idx ? total : 0);
+  r.stats.samples = total;
   if (seconds)
     *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return PT_OK;
@@ -768,13 +875,6 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   if (with_idx)
     HIP_TRY(r.scratch_idx.upload(reinterpret_cast<const uint32_t *>(stage + ray_bytes),
                                  size_t(ray_total), s));
-  HIP_TRY(r.mb_items.upload(mb.data(), m, s));
-  HIP_TRY(r.mb_blocks.upload(block_begin.data(), m + 1, s));
-  HIP_TRY(r.rgb.ensure(out_total));
-  if (final_off[m])
-    HIP_TRY(r.rgb2.ensure(final_off[m]));
-  HIP_TRY(r.counter.ensure(1));
-  HIP_TRY(hipMemsetAsync(r.counter.ptr, 0, sizeof(unsigned long long), s));
   gpu::RngParams rng{};
   rng.type = settings.rng;
   rng.samples_per = spp;
@@ -786,7 +886,24 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
     rng.dim_bound = settings.max_sample_size;
     rng.initial_dim_bound = settings.max_sample_size < 64 ? settings.max_sample_size : 64;
   }
-  HIP_TRY(hipStreamSynchronize(s)); // the staging buffer is reused below
+  // (the stream is synchronised before the staging buffer is used again)
+  const size_t sample_floats = size_t(n_img) * total * 3;
+  if (total >= kRaysWavefrontMin && (n_steps == 0 || n_steps >= 3) &&
+      sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
+    bool no_memory = false;
+    rc = rays_wavefront(r, items, act, desc, mb, settings, rng, with_idx != 0, n_steps, total,
+                        ray_total, t0, seconds, &no_memory);
+    if (!no_memory)
+      return rc;
+  }
+  HIP_TRY(r.mb_items.upload(mb.data(), m, s));
+  HIP_TRY(r.mb_blocks.upload(block_begin.data(), m + 1, s));
+  HIP_TRY(r.rgb.ensure(out_total));
+  if (final_off[m])
+    HIP_TRY(r.rgb2.ensure(final_off[m]));
+  HIP_TRY(r.counter.ensure(1));
+  HIP_TRY(hipMemsetAsync(r.counter.ptr, 0, sizeof(unsigned long long), s));
+  HIP_TRY(hipStreamSynchronize(s));
   gpu::MegaBatchParams bp{};
   bp.items = r.mb_items.ptr;
   bp.block_begin = r.mb_blocks.ptr;

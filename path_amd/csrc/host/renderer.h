@@ -236,6 +236,7 @@ struct pt_renderer {
   // batched ray-sample-spec renders: per-item descriptors and grid prefix
   pt::host::DeviceBuf<pt::gpu::MegaBatchItem> mb_items;
   pt::host::DeviceBuf<uint32_t> mb_blocks;
+  pt::host::DeviceBuf<float> ray_samples; // their per-sample values (wavefront)
 
   // adjoint buffers
   pt::host::DeviceBuf<float> adj_d_image, adj_partials, adj_out;
@@ -309,11 +310,12 @@ struct WfPipes {
   int n = 1;
 };
 // Allocate the state for n_slots paths and fill the pipelines' parameters
-// from `base` (scene, settings, rng, camera, batch, G-buffer).
+// from `base` (scene, settings, rng, camera, batch, G-buffer). Radiances go to
+// base.out_samples, or, if that is null, to r.wf_samples.
 int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
-                    uint32_t n_slots, uint64_t total_samples, bool batched,
+                    uint32_t n_slots, uint64_t total_samples, gpu::WfKind kind,
                     uint32_t trace_blocks);
-int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_blocks,
+int wavefront_run(pt_renderer &r, WfPipes &w, gpu::WfKind kind, uint32_t trace_blocks,
                   uint32_t iters_per_sync);
 int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
                  uint32_t spp, const pt_settings &settings, double *seconds);

@@ -50,7 +50,7 @@ static size_t counter_words(int n) {
 }
 
 int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
-                    uint32_t n_slots, uint64_t total_samples, bool batched,
+                    uint32_t n_slots, uint64_t total_samples, gpu::WfKind kind,
                     uint32_t trace_blocks) {
   HIP_TRY(r.wf_meta.ensure(n_slots));
   HIP_TRY(r.wf_hit_ext.ensure(n_slots));
@@ -61,9 +61,11 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
   HIP_TRY(r.wf_origin.ensure(n_slots));
   HIP_TRY(r.wf_dir.ensure(n_slots));
   HIP_TRY(r.wf_light_dir.ensure(n_slots));
+  const bool batched = kind != gpu::kWfImage;
   if (batched)
     HIP_TRY(r.wf_scene.ensure(n_slots));
-  HIP_TRY(r.wf_samples.ensure(size_t(total_samples) * 3));
+  if (!base.out_samples)
+    HIP_TRY(r.wf_samples.ensure(size_t(total_samples) * 3));
   // Pipelines have an equal share of the slots each, their own stream, queues
   // and counters: the memory-bound shade step of one overlaps the ALU-bound
   // traversal of another.
@@ -113,7 +115,8 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
     p.group_base = group_base;
     p.n_groups_total = groups_total;
     group_base += groups[h];
-    p.out_samples = r.wf_samples.ptr;
+    if (!base.out_samples)
+      p.out_samples = r.wf_samples.ptr;
     p.stack_overflow = r.wf_stack_overflow.ptr + size_t(h) * gpu::kOverflowDepth * trace_threads;
     p.overflow_stride = trace_threads;
   }
@@ -124,19 +127,19 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
 // the extension and shadow rays (one launch, which also reports the queues'
 // sizes to the host), or, with finish_blocks, take its paths to their ends.
 static hipError_t enqueue_iteration(pt_renderer &r, gpu::WfParams &p, int pipe, uint64_t iter,
-                                    bool batched, uint32_t trace_blocks, bool graph,
+                                    gpu::WfKind kind, uint32_t trace_blocks, bool graph,
                                     bool profile_events, uint32_t finish_blocks = 0) {
   hipStream_t s = r.pipe_stream(pipe);
   hipEvent_t *ev = r.ev_prof[pipe];
   hipError_t e;
   p.set = uint32_t(iter & 1);
   p.fresh = iter == 0 && !graph;
-  if ((e = gpu::launch_wf_shade(p, batched, s)) != hipSuccess)
+  if ((e = gpu::launch_wf_shade(p, kind, s)) != hipSuccess)
     return e;
   if (profile_events && (e = hipEventRecord(ev[0], s)) != hipSuccess)
     return e;
-  e = finish_blocks ? gpu::launch_wf_finish(p, batched, finish_blocks, s)
-                    : gpu::launch_wf_trace(p, batched, trace_blocks, s);
+  e = finish_blocks ? gpu::launch_wf_finish(p, kind, finish_blocks, s)
+                    : gpu::launch_wf_trace(p, kind, trace_blocks, s);
   if (e != hipSuccess)
     return e;
   if (profile_events && (e = hipEventRecord(ev[1], s)) != hipSuccess)
@@ -166,7 +169,7 @@ static hipError_t wait_report(const volatile gpu::WfReport *rep, uint32_t iterat
   return hipSuccess;
 }
 
-int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_blocks,
+int wavefront_run(pt_renderer &r, WfPipes &w, gpu::WfKind kind, uint32_t trace_blocks,
                   uint32_t iters_per_sync) {
   hipStream_t s0 = r.stream;
   const bool prof = r.profiling;
@@ -217,7 +220,7 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
       hipGraph_t graph = nullptr;
       hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
       for (uint32_t k = 0; k < iters_per_sync && e == hipSuccess; ++k)
-        e = enqueue_iteration(r, w.p[h], h, k, batched, trace_blocks, true, false);
+        e = enqueue_iteration(r, w.p[h], h, k, kind, trace_blocks, true, false);
       hipError_t e2 = hipStreamEndCapture(s, &graph);
       if (e == hipSuccess && e2 == hipSuccess)
         e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -237,7 +240,7 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
         out.launches += iters_per_sync;
       } else {
         for (uint32_t k = 0; k < iters_per_sync && out.err == hipSuccess; ++k) {
-          out.err = enqueue_iteration(r, w.p[h], h, out.launches, batched, trace_blocks, false,
+          out.err = enqueue_iteration(r, w.p[h], h, out.launches, kind, trace_blocks, false,
                                       prof);
           out.launches += 1;
         }
@@ -269,7 +272,7 @@ int wavefront_run(pt_renderer &r, WfPipes &w, bool batched, uint32_t trace_block
         const uint32_t entries = 2 * (ne + ns);
         const uint32_t blocks =
             std::min(trace_blocks, (entries + gpu::kFinishBlockPaths - 1) / gpu::kFinishBlockPaths);
-        out.err = enqueue_iteration(r, w.p[h], h, out.launches, batched, trace_blocks, false,
+        out.err = enqueue_iteration(r, w.p[h], h, out.launches, kind, trace_blocks, false,
                                     false, blocks);
         out.launches += 1;
         if (out.err != hipSuccess)
@@ -359,11 +362,11 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
   p.x_dim = x_dim;
   p.y_dim = y_dim;
   WfPipes w;
-  int rc = wavefront_alloc(r, w, p, uint32_t(slots64), total, false, trace_blocks);
+  int rc = wavefront_alloc(r, w, p, uint32_t(slots64), total, gpu::kWfImage, trace_blocks);
   if (rc != PT_OK)
     return rc;
   HIP_TRY(r.rgb.ensure(size_t(wd.num_sample_blocks) * n_pixels * 3));
-  rc = wavefront_run(r, w, false, trace_blocks, r.iters_per_sync);
+  rc = wavefront_run(r, w, gpu::kWfImage, trace_blocks, r.iters_per_sync);
   if (rc != PT_OK)
     return rc;
   hipStream_t s = r.stream;

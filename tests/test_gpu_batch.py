@@ -219,19 +219,26 @@ def _ray_items(gen_scenes, n_each, with_idx, seed=4):
 
 
 @pytest.mark.parametrize("with_idx,n_steps,spp", [(True, 5, 16), (False, 0, 16),
-                                                  (True, 3, 4096)])
+                                                  (True, 3, 4096), (True, 6, 1600),
+                                                  (False, 0, 1600), (False, 4, 1601)])
 def test_ray_batch_equals_single_renders(renderer, gen_scenes, with_idx, n_steps, spp):
     """pt_render_rays_batch (the reference datagen's per-scene InitialIdxAndDir
     + OutputPerStep renders, batched) equals pt_render of each item alone,
     bit for bit; 4096 spp over few rays spans several sample blocks per ray
-    (the second reduction pass)."""
+    (the second reduction pass); 1600 spp are enough samples for the wavefront
+    (spread over fewer sample blocks there by the work division below)."""
     from path_amd.renderer import Settings
     s = Settings()
     s.kernel_approach = "MegaKernel"
     s.back_cull_emission = 0
     items = _ray_items(gen_scenes[:4], 9 if spp > 1000 else 120, with_idx)
+    if spp == 1600:
+        s.render_work_division.force_target_samples = 1
+        s.render_work_division.forced_target_samples_per_thread = 25
     outs = renderer.render_rays_batch(items, spp, n_steps, s)
     assert renderer.last_stats().samples == sum(len(r) for _, r, _ in items) * spp
+    rays_traced = renderer.last_stats().rays
+    ref_rays = 0
     for (scene, rays, idx), got in zip(items, outs):
         if len(rays) == 0:
             assert got.size == 0
@@ -243,9 +250,11 @@ def test_ray_batch_equals_single_renders(renderer, gen_scenes, with_idx, n_steps
         else:
             ref, _ = renderer.render(scene, None, 0, 0, spp, s, rays=rays, initial_idx=idx)
             ref = ref[0]
+        ref_rays += renderer.last_stats().rays
         assert got.shape == ref.shape
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
         assert got.sum() > 0
+    assert rays_traced == ref_rays
 
 
 def test_ray_batch_rejects_mixed_specs(renderer, gen_scenes):
