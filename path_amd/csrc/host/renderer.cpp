@@ -251,6 +251,29 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
   return PT_OK;
 }
 
+// Whether the wavefront renders a MegaKernel image (the same bits: same paths,
+// same sums). It keeps its lanes busy where rays differ in length, but pays two
+// launches an iteration: it wins with many triangles, samples and vertices per
+// path. Mega-kernel / wavefront, us, at depth 1, 4, 7 and Constant 0.25:
+//   356 triangles, 2.1 M samples: 656/798, 1,767/1,417, 2,877/1,912, 2,729/2,339
+//   1,316, 1.0 M: 427/607, 1,138/1,041, 1,775/1,445, 1,903/2,028
+//   5,156, 1.0 M: 505/655, 1,296/1,134, 2,077/1,591, 1,886/2,189
+//   5,156, 4.2 M: 1,575/1,625, 4,504/3,043, 7,408/4,205, 6,440/4,637
+//   20,516, 0.5 M: 492/659, 1,166/1,182, 1,805/1,643, 2,163/2,602
+//   81,956, 4.2 M: 2,446/2,060, 7,650/3,967, 12,806/5,566, 10,717/6,342
+// 36 triangles, 4.2 M samples, depth 4: 1,428/2,091. Depth 3 with 1.6 M samples:
+// 1,497/1,339 (5,156 triangles). Paths without a depth end in a tail of short
+// iterations: with Constant 0.4 and 0.5 the sides meet at 4.2 M samples and
+// 5,156 triangles. Above 2^26 samples their radiances (12 B each) stay out of
+// memory.
+static bool wavefront_is_faster(const pt_settings &s, uint64_t samples, uint32_t n_tris) {
+  if (samples > (1u << 26))
+    return false;
+  return s.term_prob == PT_TERM_N_ITERS
+             ? s.n_iters >= 3 && samples >= (3u << 19) && n_tris >= 1024
+             : samples >= (1u << 22) && n_tris >= 4096;
+}
+
 int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
                         const pt_scene &scene, uint32_t samples_per,
                         const pt_settings &settings, bool show_progress,
@@ -347,7 +370,24 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   auto t0 = std::chrono::steady_clock::now();
   HIP_TRY(hipEventRecord(ev_start, stream));
   const float *final_rgb = nullptr;
-  if (settings.kernel_approach == PT_MEGA_KERNEL) {
+  bool wavefront = settings.kernel_approach == PT_STREAMING;
+  if (!wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
+      wavefront_is_faster(settings, uint64_t(n_pixels) * samples_per, scene_store.dev.n_tris)) {
+    bool no_memory = false;
+    uint64_t wf_rays = 0;
+    rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings, rng, x_dim, y_dim,
+                          &final_rgb, &wf_rays, &no_memory);
+    if (rc != PT_OK)
+      return rc;
+    wavefront = !no_memory;
+  } else if (wavefront) {
+    uint64_t wf_rays = 0;
+    rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings,
+                          rng, x_dim, y_dim, &final_rgb, &wf_rays);
+    if (rc != PT_OK)
+      return rc;
+  }
+  if (!wavefront) {
     WorkDivision wd;
     if (!WorkDivision::make(work_division_settings(settings.render_work_division),
                             samples_per, x_dim, y_dim, &wd))
@@ -394,12 +434,6 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
                                                  rgb2.ptr + size_t(i) * n_pixels * 3, stream));
       final_rgb = rgb2.ptr;
     }
-  } else {
-    uint64_t wf_rays = 0;
-    rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings,
-                          rng, x_dim, y_dim, &final_rgb, &wf_rays);
-    if (rc != PT_OK)
-      return rc;
   }
   if (out.type == PT_OUTPUT_BGRA) {
     HIP_TRY(bgra.ensure(n_pixels));
@@ -442,7 +476,7 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, ev_start, ev_stop));
   stats.kernel_ms = ms;
-  stats.rays = settings.kernel_approach == PT_STREAMING
+  stats.rays = wavefront
                    ? stats.ext_rays + stats.shadow_rays
                    : rays_traced;
   stats.samples = uint64_t(samples_per) * n_pixels;

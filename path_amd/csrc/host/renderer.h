@@ -236,7 +236,9 @@ struct pt_renderer {
   // batched ray-sample-spec renders: per-item descriptors and grid prefix
   pt::host::DeviceBuf<pt::gpu::MegaBatchItem> mb_items;
   pt::host::DeviceBuf<uint32_t> mb_blocks;
-  pt::host::DeviceBuf<float> ray_samples; // their per-sample values (wavefront)
+  // per-sample values of wavefront renders other than the Streaming
+  // integrator's (ray batches, images the mega-kernel hands over)
+  pt::host::DeviceBuf<float> ray_samples;
 
   // adjoint buffers
   pt::host::DeviceBuf<float> adj_d_image, adj_partials, adj_out;
@@ -330,10 +332,13 @@ int render_adjoint(pt_renderer &r, const pt_scene &scene, const float film_to_wo
                    float *grad_emission, double *seconds);
 // Wavefront ("Streaming") integrator; writes the final per-pixel FloatRGB
 // (already divided by samples_per) into a device buffer owned by the renderer.
+// With no_memory it stands in for the mega-kernel: the path pool is its own,
+// the last Streaming render's samples are kept (pt_last_render_fp64), and *no_memory
+// is set, and nothing rendered, if its buffers do not fit the device.
 int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
                      const gpu::DeviceScene &scene, uint32_t samples_per,
                      const pt_settings &settings, const gpu::RngParams &rng,
                      uint32_t x_dim, uint32_t y_dim, const float **final_rgb,
-                     uint64_t *rays_out);
+                     uint64_t *rays_out, bool *no_memory = nullptr);
 } // namespace host
 } // namespace pt

@@ -71,3 +71,33 @@ def test_batch_equals_single_renders(renderer, spp, forced):
         assert np.array_equal(np.asarray(img).reshape(mega.shape).view(np.uint32),
                               mega.view(np.uint32))
         assert np.isfinite(gb).all() and np.abs(gb).sum() > 0
+
+
+# either side of the sizes at which MegaKernel images run on the wavefront's
+# kernels: samples, depth; roulette from 4.2 M samples; ragged images
+@pytest.mark.parametrize("x,y,spp,term,iters,handed_over", [
+    (261, 211, 29, "NIters", 3, True), (256, 256, 24, "NIters", 2, False),
+    (256, 255, 24, "NIters", 4, False), (256, 256, 64, "Constant", 0, True),
+    (256, 255, 64, "Constant", 0, False)])
+def test_megakernel_images_on_the_wavefront(renderer, benchmark_scene, x, y, spp, term, iters,
+                                            handed_over):
+    scene, ftw = benchmark_scene
+    small = _settings("Streaming", "NIters", "Sobel")
+    renderer.render(scene, ftw, 20, 15, 4, small)
+    resummed = renderer.last_render_fp64(20, 15)
+    s = _settings("MegaKernel", term, "Sobel")
+    s.n_iters = iters
+    s.max_num_samples_per_launch = 100  # the Streaming integrator's, not this call's
+    try:
+        renderer.set_megakernel_split(False)
+        ref, _ = renderer.render(scene, ftw, x, y, spp, s)
+        assert renderer.last_stats().mega_launches > 0
+        rays = renderer.last_stats().rays
+    finally:
+        renderer.set_megakernel_split(True)
+    img, _ = renderer.render(scene, ftw, x, y, spp, s)
+    assert (renderer.last_stats().mega_launches == 0) == handed_over
+    assert renderer.last_stats().rays == rays
+    assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
+    # the last Streaming render can still be summed in FP64
+    assert np.array_equal(renderer.last_render_fp64(20, 15), resummed)
