@@ -122,9 +122,9 @@ PT_INLINE bool hit_before(T t, uint32_t idx, T best_t, uint32_t best_idx) {
 // on the 82k-triangle scene's glass) walked the whole tree alone for 80 ms, of
 // an image that takes 18.
 template <class T> PT_INLINE bool ray_can_hit(const Ray<T> &r) {
-  const T z = T(0);
-  return fma_(r.d.x, z, fma_(r.d.y, z, r.d.z * z)) == z && r.o.x == r.o.x && r.o.y == r.o.y &&
-         r.o.z == r.o.z;
+  const T z = T(0); // times an infinity or NaN: NaN
+  const T bad_d = fma_(r.d.x, z, fma_(r.d.y, z, r.d.z * z));
+  return !__builtin_isunordered(r.o.x, r.o.y) && !__builtin_isunordered(r.o.z, bad_d);
 }
 
 // reference: include/intersect/intersection.h:17-20
