@@ -334,9 +334,14 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
     return set_error(PT_ERR_INVALID, "unknown kernel approach");
 
   HIP_TRY(hipSetDevice(device));
+  // (the last scene with a generation's stamp: it is in device memory)
+  const pt_scene *had_scene = cached_scene;
+  const uint64_t had_gen = cached_gen, had_mat_gen = cached_mat_gen;
   int rc = ensure_scene(scene, &settings);
   if (rc != PT_OK)
     return rc;
+  const bool resident =
+      had_scene == cached_scene && had_gen == cached_gen && had_mat_gen == cached_mat_gen;
   gpu::RngParams rng{};
   rng.type = settings.rng;
   rng.samples_per = samples_per;
@@ -363,7 +368,10 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
                                              " out of range");
     HIP_TRY(scratch_idx.upload(spec.initial_idx, spec.n_rays, stream));
   }
-  HIP_TRY(hipStreamSynchronize(stream));
+  // Uploads from host memory end here, before anything is timed. Without any,
+  // the render goes straight on (64 x 64 at 4 spp: the wait was 24 of 142 us).
+  if (!resident || spec.type != PT_SAMPLE_SQUARE_IMAGE)
+    HIP_TRY(hipStreamSynchronize(stream));
 
   stats = pt_render_stats{};
   stats.profiled = profiling ? 1u : 0u;
@@ -446,8 +454,8 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   const size_t image_bytes = size_t(n_pixels) * (out.type == PT_OUTPUT_BGRA ? 4 : 12);
   const uint32_t n_images = per_step ? out.n_steps : 1;
   const bool host_out = out.type != PT_OUTPUT_DEVICE_FLOAT_RGB;
-  if (host_out)
-    HIP_TRY(out_stage.ensure(image_bytes * n_images + sizeof(unsigned long long)));
+  const size_t staged_bytes = host_out ? image_bytes * n_images : 0;
+  HIP_TRY(out_stage.ensure(staged_bytes + sizeof(unsigned long long)));
   char *stage = static_cast<char *>(out_stage.ptr);
   if (out.type == PT_OUTPUT_BGRA)
     HIP_TRY(hipMemcpyAsync(stage, bgra.ptr, image_bytes, hipMemcpyDeviceToHost, stream));
@@ -457,12 +465,8 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
     HIP_TRY(hipMemcpyAsync(stage, final_rgb, image_bytes * n_images, hipMemcpyDeviceToHost,
                            stream));
   unsigned long long rays_traced = 0;
-  if (host_out)
-    HIP_TRY(hipMemcpyAsync(stage + image_bytes * n_images, counter.ptr, sizeof(rays_traced),
-                           hipMemcpyDeviceToHost, stream));
-  else
-    HIP_TRY(hipMemcpyAsync(&rays_traced, counter.ptr, sizeof(rays_traced),
-                           hipMemcpyDeviceToHost, stream));
+  HIP_TRY(hipMemcpyAsync(stage + staged_bytes, counter.ptr, sizeof(rays_traced),
+                         hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
   if (host_out) {
     if (per_step)
@@ -470,8 +474,8 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
         std::memcpy(out.per_step[i], stage + image_bytes * i, image_bytes);
     else
       std::memcpy(out.data, stage, image_bytes);
-    std::memcpy(&rays_traced, stage + image_bytes * n_images, sizeof(rays_traced));
   }
+  std::memcpy(&rays_traced, stage + staged_bytes, sizeof(rays_traced));
   auto t1 = std::chrono::steady_clock::now();
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, ev_start, ev_stop));
