@@ -146,8 +146,8 @@ hipError_t launch_nrc_paths(const NrcParams &p, hipStream_t s);
 // Per pixel (pixel-centre camera ray): features of the first hit, the
 // emission seen there in base and weight 1 (all zero for a miss).
 hipError_t launch_nrc_first_vertex(const NrcParams &p, hipStream_t s);
-// out_rgb[pixel] = sum_s (base + weight * max(pred[0..3], 0)) / spp with pred
-// rows of 16 floats.
+// out_rgb[pixel] = sum_s (base + weight * max(pred, 0)) / spp, all three
+// arrays [pixel][sample][3].
 hipError_t launch_nrc_combine(const float *base, const float *weight, const float *pred,
                               uint32_t n_pixels, uint32_t spp, float *out_rgb,
                               hipStream_t s);

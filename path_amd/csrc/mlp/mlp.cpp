@@ -127,7 +127,7 @@ static GemmArgs gemm_args(const bf16 *A, uint32_t lda, const bf16 *B, uint32_t l
 
 int pt_mlp::forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad, hipStream_t on) {
   hipStream_t stream = on ? on : this->stream;
-  HIP_TRY(pred.ensure(size_t(rows_pad) * kOutPad));
+  HIP_TRY(pred.ensure(size_t(rows_pad) * kOut));
   if (fused_forward) {
     MlpTileArgs t{};
     t.feat = d_feat;
@@ -137,6 +137,7 @@ int pt_mlp::forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad, h
     HIP_TRY(launch_mlp_tile(t, rows_pad, false, stream));
     return PT_OK;
   }
+  HIP_TRY(pred_pad.ensure(size_t(rows_pad) * kOutPad));
   HIP_TRY(x0.ensure(size_t(rows_pad) * kInPad));
   for (auto &a : act)
     HIP_TRY(a.ensure(size_t(rows_pad) * kWidth));
@@ -151,9 +152,10 @@ int pt_mlp::forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad, h
                           kEpiReluBf16, stream));
       in = out;
     } else {
-      HIP_TRY(launch_gemm(gemm_args(in, kWidth, w, kWidth, rows_pad, kOutPad, kWidth, pred.ptr,
-                                    kOutPad),
+      HIP_TRY(launch_gemm(gemm_args(in, kWidth, w, kWidth, rows_pad, kOutPad, kWidth,
+                                    pred_pad.ptr, kOutPad),
                           kEpiF32, stream));
+      HIP_TRY(launch_compact_pred(pred_pad.ptr, rows_pad, pred.ptr, stream));
     }
   }
   return PT_OK;
@@ -293,10 +295,7 @@ int pt_mlp_forward(pt_mlp *m, const float *features, uint32_t n, float *out) {
   int rc = m->forward_device(m->feat.ptr, n, rp);
   if (rc != PT_OK)
     return rc;
-  // compact to n x 3 on the device (reuses the front of the target buffer)
-  HIP_TRY(m->targ.ensure(size_t(rp) * kOut));
-  HIP_TRY(launch_compact_pred(m->pred.ptr, n, m->targ.ptr, m->stream));
-  HIP_TRY(hipMemcpyAsync(out, m->targ.ptr, size_t(n) * kOut * 4, hipMemcpyDeviceToHost,
+  HIP_TRY(hipMemcpyAsync(out, m->pred.ptr, size_t(n) * kOut * 4, hipMemcpyDeviceToHost,
                          m->stream));
   HIP_TRY(hipStreamSynchronize(m->stream));
   return PT_OK;

@@ -19,6 +19,7 @@ struct pt_mlp {
   // per-batch buffers (grow-only, rows padded to kRowAlign)
   pt::host::DeviceBuf<float> feat, targ, pred;
   pt::host::DeviceBuf<pt::mlp::bf16> x0, act[2]; // layer-by-layer forward
+  pt::host::DeviceBuf<float> pred_pad;           // and its padded output
   // training: layer inputs and output gradients in fragment order, activation
   // bits, per-tile and per-split partial sums
   pt::host::DeviceBuf<uint16_t> a_frag, g_frag;
@@ -34,7 +35,7 @@ struct pt_mlp {
   bool init(int dev, uint64_t seed, std::string *err);
   int ensure_training(uint32_t rows_pad, uint32_t steps);
   // Forward on device features (n rows; rows up to rows_pad count as zero
-  // features): pred[rows_pad x 16] fp32, by the fused kernel unless disabled.
+  // features): pred[rows_pad x 3] fp32, by the fused kernel unless disabled.
   int forward_device(const float *d_feat, uint32_t n, uint32_t rows_pad,
                      hipStream_t on = nullptr);
   // Forward, loss, backward of a batch of n rows: per-split gradients in

@@ -285,8 +285,8 @@ __global__ __launch_bounds__(256, 2) void k_mlp_tile(MlpTileArgs a) {
           d = f2bf(2.f * e / den * inv);
         }
         D[row * kDStride + l32] = d;
-      } else if (l32 < kOutPad) {
-        a.pred[size_t(row0 + row) * kOutPad + l32] = o[r];
+      } else if (l32 < kOut) {
+        a.pred[size_t(row0 + row) * kOut + l32] = o[r];
       }
     }
     if constexpr (kTrain) {

@@ -73,7 +73,7 @@ struct MlpTileArgs {
   uint64_t seed;
   uint32_t n;
   const uint16_t *w_frag, *wt_frag;
-  float *pred;              // inference: [rows_pad x 16]
+  float *pred;              // inference: [rows_pad x 3]
   // training
   uint16_t *a_frag, *g_frag; // layer l's input / output gradient at l * layer_stride
   size_t layer_stride;       // rows_pad * 256
