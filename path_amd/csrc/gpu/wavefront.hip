@@ -9,7 +9,7 @@
 // device-scope atomics are the expensive operation on this chip.
 //
 // Batched renders (many scenes in one launch sequence) are the same kernels
-// instantiated with kBatch: every slot also carries its scene, whose BVH,
+// instantiated for another WfKind: every slot also carries its scene, whose BVH,
 // shading records, materials and lights are addressed through offsets into
 // concatenated arrays.
 // reference semantics: include/render/detail/integrate_image/streaming/run_impl.h:155-460
