@@ -32,7 +32,8 @@ constexpr uint32_t kKSteps = kWidth / 16;
 constexpr uint32_t kColBlocks = kWidth / 32;
 constexpr uint32_t kLayerFrags = kColBlocks * kKSteps; // fragments of a hidden layer
 // weight fragments in flight ahead of their MFMAs (2 / 3 / 4: 611 / 613 / 606
-// us per 2^20 queries, 270 / 267 / 266 us per training step of 65,536 rows)
+// us per 2^20 queries, 270 / 267 / 266 us per training step of 65,536 rows with
+// cached stores)
 constexpr uint32_t kWAhead = 3;
 
 // Row of the training set that row i of a step draws (SplitMix64).
@@ -59,8 +60,18 @@ __device__ __forceinline__ bf16x8_t column_frag(const uint16_t *tile, uint32_t s
   return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// Batches of at least kStreamRows rows write A and G past the caches and read
+// them back the same way: what one kernel writes (0.15 GB there, 0.4 GB at
+// 65,536 rows) is evicted before the next reads it, and takes the weights with
+// it. Training step, us, cached / stores streamed / loads too: 16,384 rows 91 /
+// 94 / 94; 24,576: 111 / 116 / 115; 32,768: 139 / 139 / 129; 65,536: 258 / 242 /
+// 216; 131,072: 497 / 440 / 395.
+constexpr uint32_t kStreamRows = 24576;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
 // The tile's fragments for the weight gradient: wave w writes the column
-// blocks 2 w and 2 w + 1.
+// blocks 2 w and 2 w + 1. (Tiles of more than 32 rows are those of batches of
+// at least kStreamRows.)
 template <uint32_t kI>
 __device__ __forceinline__ void store_column_frags(const uint16_t *X, uint16_t *__restrict__ dst,
                                                    uint32_t wave) {
@@ -70,8 +81,13 @@ __device__ __forceinline__ void store_column_frags(const uint16_t *X, uint16_t *
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
       const uint32_t cb = 2 * wave + j;
-      *reinterpret_cast<bf16x8_t *>(dst + (size_t(rb) * kColBlocks + cb) * kFrag + lane * 8u) =
-          column_frag(X, kXStride, rb, cb);
+      auto *at = reinterpret_cast<bf16x8_t *>(dst + (size_t(rb) * kColBlocks + cb) * kFrag +
+                                              lane * 8u);
+      const bf16x8_t v = column_frag(X, kXStride, rb, cb);
+      if constexpr (kI > 1)
+        __builtin_nontemporal_store(v, at);
+      else
+        *at = v;
     }
 }
 
@@ -204,7 +220,7 @@ template <uint32_t kI> constexpr size_t tile_lds(bool train) {
 // Inference is bound by the matrix cores: 2^20 queries 0.61 ms, 1.35 PFLOP/s
 // (0.94 ms with row-major weights and two-byte stores of the encoding); a
 // large bf16 library product reaches 1.23 on the same card. Training at
-// 65,536 rows: 144 us for 75 us of matrix work and 0.4 GB written (one GEMM
+// 65,536 rows: 130 us for 75 us of matrix work and 0.4 GB written (one GEMM
 // launch per layer and direction with row-major and transposed copies took
 // 420 us and moved 2.2 GB).
 template <uint32_t kI, bool kTrain>
@@ -365,10 +381,10 @@ __global__ __launch_bounds__(256, 2) void k_mlp_tile(MlpTileArgs a) {
 // rows, the chip's 256 CUs many tiles. Training step, us, tiles of 32 / 64 /
 // 128 rows: 3,001 rows 60 / 69 / 93; 16,384: 93 / 95 / 117; 24,576: 113 / 113 /
 // 131; 32,768: 151 / 142 / 157; 49,152: 210+ / 203 / 210; 65,536: 313 / 276 /
-// 267. Inference: 4,096 rows 12 / 17 / 26; 16,384: 20 / 18 / 27; 65,536: 66 /
+// 267 (all with cached stores and loads). Inference: 4,096 rows 12 / 17 / 26; 16,384: 20 / 18 / 27; 65,536: 66 /
 // 52 / 45; 2^20: 879 / 677 / 607.
 uint32_t mlp_tile_rows(uint32_t rows_pad) {
-  return rows_pad < 24576u ? 32u : rows_pad < 57344u ? 64u : 128u;
+  return rows_pad < kStreamRows ? 32u : rows_pad < 57344u ? 64u : 128u;
 }
 
 template <uint32_t kI> static hipError_t launch_tile(const MlpTileArgs &a, uint32_t rows_pad,
@@ -399,8 +415,9 @@ hipError_t launch_mlp_tile(const MlpTileArgs &a, uint32_t rows_pad, bool train, 
 // operands are read from memory exactly once. Stages of 32 rows (32 KB, both
 // operands contiguous in memory) go through registers two stages ahead into a
 // double-buffered LDS tile. Bound by HBM: 65,536 rows read 0.40 GB and write
-// 66 MB of partials in 108 us, 4.3 TB/s where a large copy reaches 4.7 (128 x
-// 128 tiles and 128 splits took 140 us, and 43 us to sum).
+// 66 MB of partials in 82 us, 5.7 TB/s where a large copy reaches 4.7 (108 us
+// with cached loads; 128 x 128 tiles and 128 splits took 140 us, and 43 us to
+// sum).
 // The first blocks of the grid do the small sums: the output layer's partial
 // gradients (one block per output) and the loss.
 // ---------------------------------------------------------------------------
@@ -435,6 +452,7 @@ __device__ __forceinline__ void sum_tiles(const MlpWgradArgs &a) {
   }
 }
 
+template <bool kStream>
 __global__ __launch_bounds__(512, 2) void k_mlp_wgrad(MlpWgradArgs a) {
   if (blockIdx.x < kWgExtra) { // whole block
     sum_tiles(a);
@@ -466,7 +484,15 @@ __global__ __launch_bounds__(512, 2) void k_mlp_wgrad(MlpWgradArgs a) {
   };
   auto fetch = [&](uint32_t s) __attribute__((always_inline)) {
     const size_t o = size_t(min(s, stages - 1)) * (kStage / 8) + t;
-    return Regs{g[o], g[o + 512], x[o], x[o + 512]};
+    if constexpr (kStream) {
+      auto load = [](const uint4 *p) __attribute__((always_inline)) {
+        return __builtin_bit_cast(
+            uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p)));
+      };
+      return Regs{load(g + o), load(g + o + 512), load(x + o), load(x + o + 512)};
+    } else {
+      return Regs{g[o], g[o + 512], x[o], x[o + 512]};
+    }
   };
   Regs v0 = fetch(s0), v1 = fetch(s0 + 1);
   auto step = [&](uint32_t s, Regs &r, uint16_t *tile) __attribute__((always_inline)) {
@@ -524,7 +550,11 @@ uint32_t mlp_wgrad_splits(uint32_t rows_pad) {
 hipError_t launch_mlp_wgrad(const MlpWgradArgs &a, hipStream_t s) {
   if (a.rows_pad % kRowAlign || a.splits == 0)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(kWgExtra + kHidden * a.splits), dim3(512), 0, s, a);
+  const dim3 grid(kWgExtra + kHidden * a.splits);
+  if (a.rows_pad >= kStreamRows)
+    hipLaunchKernelGGL(k_mlp_wgrad<true>, grid, dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_mlp_wgrad<false>, grid, dim3(512), 0, s, a);
   return hipGetLastError();
 }
 
