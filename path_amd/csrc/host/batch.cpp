@@ -888,8 +888,8 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   }
   // (the stream is synchronised before the staging buffer is used again)
   const size_t sample_floats = size_t(n_img) * total * 3;
-  if (total >= kRaysWavefrontMin && (n_steps == 0 || n_steps >= 3) &&
-      sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
+  if (r.mega_split && !r.profiling && total >= kRaysWavefrontMin &&
+      (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
     bool no_memory = false;
     rc = rays_wavefront(r, items, act, desc, mb, settings, rng, with_idx != 0, n_steps, total,
                         ray_total, t0, seconds, &no_memory);

@@ -1,0 +1,95 @@
+"""Host side of the renders (which kernels a call takes, what memory it holds,
+what an error return leaves behind) on the CPU: the library's host sources
+linked with a HIP runtime that runs nothing (native/fake_hip.cpp)."""
+import concurrent.futures as cf
+import ctypes as C
+import gc
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from path_amd import _lib as L
+from path_amd import build
+
+FAKE = Path(__file__).resolve().parent / "native" / "fake_hip.cpp"
+
+
+@pytest.fixture(scope="module")
+def host_library(tmp_path_factory):
+    d = tmp_path_factory.mktemp("host")
+    srcs = [build.CSRC / s for s in build.SOURCES if s.endswith(".cpp")] + [FAKE]
+
+    def compiled(src):
+        obj = d / (src.name + ".o")
+        subprocess.run([build.HIPCC, "-x", "hip", "--cuda-host-only", "-O1", "-std=c++20", "-fPIC",
+                        "-ffp-contract=off", "-march=x86-64-v3", f"--offload-arch={build.ARCH}",
+                        "-c", str(src), "-o", str(obj)], check=True, capture_output=True)
+        return str(obj)
+    with cf.ThreadPoolExecutor(8) as ex:
+        objs = list(ex.map(compiled, srcs))
+    so = d / "libhost.so"
+    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-pthread", "-o", str(so), *objs],
+                   check=True)
+    lib = C.CDLL(str(so))
+    for name, (res, args) in L.SIGNATURES.items():
+        if hasattr(lib, name):
+            getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
+    for name in ("live", "largest", "launches", "most", "in_flight"):
+        getattr(lib, "fake_" + name).restype = C.c_uint64
+    lib.fake_limit.argtypes = [C.c_uint64]
+    return lib
+
+
+@pytest.fixture
+def fake(host_library, monkeypatch):
+    """The package on that library; every object of the test is gone before
+    the real one is back."""
+    monkeypatch.setattr(L, "_lib", host_library)
+    host_library.fake_reset()
+    yield host_library
+    gc.collect()
+
+
+def _settings(**kw):
+    from path_amd.renderer import Settings
+    s = Settings()
+    s.kernel_approach, s.rng = "MegaKernel", "Uniform"
+    s.term_prob, s.n_iters = "NIters", 5
+    for k, v in kw.items():
+        setattr(s, k, v)
+    return s
+
+
+def _scene(n_tris):
+    from path_amd.renderer import Scene, material
+    rng = np.random.default_rng(1)
+    v = rng.uniform(-1, 1, (n_tris, 1, 3)) + rng.uniform(-0.05, 0.05, (n_tris, 3, 3))
+    s = Scene()
+    s.add_mesh(v.reshape(-1, 9).astype(np.float32), np.zeros(n_tris, np.uint32),
+               [material("Diffuse", diffuse=(0.5,) * 3, emission=(1, 1, 1))])
+    return s
+
+
+FTW = np.eye(3, 4, dtype=np.float32).ravel()
+
+
+def _rays(n, seed=0):
+    return np.random.default_rng(seed).uniform(-1, 1, (n, 6)).astype(np.float32)
+
+
+# what a call above the hand-over's sizes runs on
+@pytest.mark.parametrize("control,wavefront", [
+    (lambda r: None, True),
+    (lambda r: r.set_megakernel_split(False), False),
+    (lambda r: r.set_profiling(True), False)])
+def test_controls_of_the_hand_over(fake, control, wavefront):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(1100)
+    control(r)
+    r.render(scene, FTW, 256, 256, 24, _settings())
+    assert (fake.fake_launches(b"mega") == 0) == wavefront
+    r.render_rays_batch([(scene, _rays(4096), None)], 64, 0, _settings())
+    assert (fake.fake_launches(b"mega_batch") == 0) == wavefront
+    assert (fake.fake_launches(b"wf_trace") > 0) == wavefront
