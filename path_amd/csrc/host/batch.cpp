@@ -676,9 +676,10 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
   return PT_OK;
 }
 
-// The wavefront traces a batch's rays from this many samples on, and of three
-// steps or more: the mega-kernel's waves wait for their longest path, the
-// wavefront pays two launches an iteration. Whole calls, us, mega-kernel /
+// The wavefront traces a batch's rays from this many samples on (and, where
+// launches are limited, this many in each), and of three steps or more: the
+// mega-kernel's waves wait for their longest path, the wavefront pays two
+// launches an iteration. Whole calls, us, mega-kernel /
 // wavefront, six steps: 89,600 samples 1,102 / 1,015, 192,000: 1,292 / 1,356,
 // 384,000: 1,684 / 1,321, 1.15 M: 3,387 / 2,479; no steps: 240,000: 1,449 /
 // 1,237, 768,000: 2,305 / 1,834; three steps, 576,000: 1,323 / 1,051; one step,
@@ -689,7 +690,7 @@ constexpr size_t kRaysWavefrontBytes = size_t(4) << 30;
 
 // The wavefront's part of render_rays_batch: scenes, rays and indices are on the
 // device. Values are summed like the mega-kernel's, so they are the same bits.
-// *no_memory is set, and nothing done, if its buffers do not fit the device.
+// no_memory is set, and nothing done, if its buffers do not fit the device.
 static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
                           const std::vector<uint32_t> &act,
                           const std::vector<gpu::SceneDesc> &desc,
@@ -697,12 +698,12 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
                           const gpu::RngParams &rng, bool with_idx, uint32_t n_steps,
                           uint64_t total, uint64_t n_rays,
                           std::chrono::steady_clock::time_point t0, double *seconds,
-                          bool *no_memory) {
+                          HandOver *hand_over) {
   hipStream_t s = r.stream;
   const uint32_t n_img = n_steps ? n_steps : 1, m = uint32_t(act.size());
   if (r.ray_samples.ensure(size_t(n_img) * total * 3) != hipSuccess) {
     (void)hipGetLastError();
-    *no_memory = true;
+    hand_over->no_memory = true;
     return PT_OK;
   }
   HIP_TRY(r.rgb.ensure(size_t(n_img) * n_rays * 3));
@@ -715,13 +716,13 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
   p.batch.n_steps = n_steps;
   p.out_samples = r.ray_samples.ptr;
   // (max_num_samples_per_launch is the Streaming integrator's setting)
-  const uint64_t slots = std::min<uint64_t>(1u << 22, total);
+  const uint64_t slots = hand_over->max_paths;
   const uint32_t trace_blocks = uint32_t(r.n_cus) * r.trace_blocks_for(true);
   WfPipes w;
   int rc = wavefront_alloc(r, w, p, uint32_t(slots), total, gpu::kWfRays, trace_blocks);
   if (rc != PT_OK) {
     (void)hipGetLastError();
-    *no_memory = true;
+    hand_over->no_memory = true;
     return PT_OK;
   }
   BatchReduction red;
@@ -888,12 +889,13 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   }
   // (the stream is synchronised before the staging buffer is used again)
   const size_t sample_floats = size_t(n_img) * total * 3;
-  if (r.mega_split && !r.profiling && total >= kRaysWavefrontMin &&
+  HandOver hand_over{
+      hand_over_paths(total, block_begin[m], settings.max_blocks_per_launch_gpu)};
+  if (r.mega_split && !r.profiling && hand_over.max_paths >= kRaysWavefrontMin &&
       (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
-    bool no_memory = false;
     rc = rays_wavefront(r, items, act, desc, mb, settings, rng, with_idx != 0, n_steps, total,
-                        ray_total, t0, seconds, &no_memory);
-    if (!no_memory)
+                        ray_total, t0, seconds, &hand_over);
+    if (!hand_over.no_memory)
       return rc;
   }
   HIP_TRY(r.mb_items.upload(mb.data(), m, s));

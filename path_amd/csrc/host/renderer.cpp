@@ -265,9 +265,10 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
 // 1,497/1,339 (5,156 triangles). Paths without a depth end in a tail of short
 // iterations: with Constant 0.4 and 0.5 the sides meet at 4.2 M samples and
 // 5,156 triangles. Above 2^26 samples their radiances (12 B each) stay out of
-// memory.
-static bool wavefront_is_faster(const pt_settings &s, uint64_t samples, uint32_t n_tris) {
-  if (samples > (1u << 26))
+// memory. Launches limited to fewer than 2^20 paths stay with the mega-kernel.
+static bool wavefront_is_faster(const pt_settings &s, uint64_t samples, uint64_t paths,
+                                uint32_t n_tris) {
+  if (samples > (1u << 26) || paths < (1u << 20))
     return false;
   return s.term_prob == PT_TERM_N_ITERS
              ? s.n_iters >= 3 && samples >= (3u << 19) && n_tris >= 1024
@@ -379,15 +380,27 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   HIP_TRY(hipEventRecord(ev_start, stream));
   const float *final_rgb = nullptr;
   bool wavefront = settings.kernel_approach == PT_STREAMING;
+  WorkDivision wd;
+  if (!wavefront) {
+    if (!WorkDivision::make(work_division_settings(settings.render_work_division),
+                            samples_per, x_dim, y_dim, &wd))
+      return set_error(PT_ERR_INVALID, "invalid render work division settings");
+    if (wd.block_size > 1024)
+      return set_error(PT_ERR_INVALID, "block_size above 1024");
+  }
+  const uint64_t samples = uint64_t(n_pixels) * samples_per;
+  const uint64_t paths = wavefront ? 0
+                                   : hand_over_paths(samples, wd.total_num_blocks(),
+                                                     settings.max_blocks_per_launch_gpu);
   if (!wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
-      wavefront_is_faster(settings, uint64_t(n_pixels) * samples_per, scene_store.dev.n_tris)) {
-    bool no_memory = false;
+      wavefront_is_faster(settings, samples, paths, scene_store.dev.n_tris)) {
+    HandOver hand_over{paths};
     uint64_t wf_rays = 0;
     rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings, rng, x_dim, y_dim,
-                          &final_rgb, &wf_rays, &no_memory);
+                          &final_rgb, &wf_rays, &hand_over);
     if (rc != PT_OK)
       return rc;
-    wavefront = !no_memory;
+    wavefront = !hand_over.no_memory;
   } else if (wavefront) {
     uint64_t wf_rays = 0;
     rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings,
@@ -396,12 +409,6 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
       return rc;
   }
   if (!wavefront) {
-    WorkDivision wd;
-    if (!WorkDivision::make(work_division_settings(settings.render_work_division),
-                            samples_per, x_dim, y_dim, &wd))
-      return set_error(PT_ERR_INVALID, "invalid render work division settings");
-    if (wd.block_size > 1024)
-      return set_error(PT_ERR_INVALID, "block_size above 1024");
     const size_t image_floats = size_t(wd.num_sample_blocks) * n_pixels * 3;
     HIP_TRY(rgb.ensure(image_floats * (per_step ? out.n_steps : 1)));
     gpu::MegaParams p{};

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <memory>
 #include <string>
 
@@ -332,13 +333,27 @@ int render_adjoint(pt_renderer &r, const pt_scene &scene, const float film_to_wo
                    float *grad_emission, double *seconds);
 // Wavefront ("Streaming") integrator; writes the final per-pixel FloatRGB
 // (already divided by samples_per) into a device buffer owned by the renderer.
-// With no_memory it stands in for the mega-kernel: the path pool is its own,
-// the last Streaming render's samples are kept (pt_last_render_fp64), and *no_memory
+// With hand_over it stands in for the mega-kernel: the path pool is max_paths,
+// the last Streaming render's samples are kept (pt_last_render_fp64), and no_memory
 // is set, and nothing rendered, if its buffers do not fit the device.
+struct HandOver {
+  uint64_t max_paths;
+  bool no_memory = false;
+};
+// Paths of the pool of work handed over: at most kHandOverPool, and at most the
+// samples that a mega-kernel launch of max_blocks (0: all) of its grid's blocks
+// has, so that a limit on launches keeps bounding them (each of the wavefront's
+// takes its paths one vertex further).
+constexpr uint64_t kHandOverPool = 1u << 22;
+inline uint64_t hand_over_paths(uint64_t samples, uint64_t blocks, uint32_t max_blocks) {
+  if (max_blocks != 0 && max_blocks < blocks)
+    samples = uint64_t(double(samples) / double(blocks) * max_blocks);
+  return std::min(samples, kHandOverPool);
+}
 int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
                      const gpu::DeviceScene &scene, uint32_t samples_per,
                      const pt_settings &settings, const gpu::RngParams &rng,
                      uint32_t x_dim, uint32_t y_dim, const float **final_rgb,
-                     uint64_t *rays_out, bool *no_memory = nullptr);
+                     uint64_t *rays_out, HandOver *hand_over = nullptr);
 } // namespace host
 } // namespace pt

@@ -337,7 +337,7 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
                      const gpu::DeviceScene &scene, uint32_t samples_per,
                      const pt_settings &settings, const gpu::RngParams &rng,
                      uint32_t x_dim, uint32_t y_dim, const float **final_rgb,
-                     uint64_t *rays_out, bool *no_memory) {
+                     uint64_t *rays_out, HandOver *hand_over) {
   if (spec.type != PT_SAMPLE_SQUARE_IMAGE)
     return set_error(PT_ERR_UNSUPPORTED,
                      "the Streaming integrator takes SquareImage sample specs");
@@ -348,7 +348,7 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
     return set_error(PT_ERR_INVALID, "invalid render work division settings");
   const uint64_t n_pixels = uint64_t(x_dim) * y_dim;
   const uint64_t total = n_pixels * samples_per;
-  uint64_t slots64 = no_memory ? 1u << 22 : settings.max_num_samples_per_launch;
+  uint64_t slots64 = hand_over ? hand_over->max_paths : settings.max_num_samples_per_launch;
   if (slots64 == 0)
     return set_error(PT_ERR_INVALID, "max_num_samples_per_launch must be positive");
   if (slots64 > total)
@@ -361,19 +361,19 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
   std::memcpy(p.film_to_world, spec.film_to_world, sizeof(p.film_to_world));
   p.x_dim = x_dim;
   p.y_dim = y_dim;
-  if (no_memory) {
+  if (hand_over) {
     if (r.ray_samples.ensure(size_t(total) * 3) != hipSuccess) {
       (void)hipGetLastError();
-      *no_memory = true;
+      hand_over->no_memory = true;
       return PT_OK;
     }
     p.out_samples = r.ray_samples.ptr;
   }
   WfPipes w;
   int rc = wavefront_alloc(r, w, p, uint32_t(slots64), total, gpu::kWfImage, trace_blocks);
-  if (rc != PT_OK && no_memory) {
+  if (rc != PT_OK && hand_over) {
     (void)hipGetLastError();
-    *no_memory = true;
+    hand_over->no_memory = true;
     return PT_OK;
   }
   if (rc != PT_OK)
@@ -394,7 +394,7 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
   }
   *final_rgb = out;
   *rays_out = r.stats.ext_rays + r.stats.shadow_rays;
-  if (!no_memory) {
+  if (!hand_over) {
     r.last_wf_x = x_dim;
     r.last_wf_y = y_dim;
     r.last_wf_spp = samples_per;

@@ -23,10 +23,11 @@ namespace {
 struct Fake {
   std::mutex m;
   std::map<const char *, size_t> device, pinned;
-  std::map<std::string, uint64_t> launches, most; // count; largest size argument
+  std::map<std::string, uint64_t> launches;
   std::map<hipStream_t, int> reads;               // copies out of pinned memory
   std::string failing;
   size_t limit = size_t(1) << 60, live = 0, largest = 0;
+  uint64_t pool = 0; // paths of the wavefront renders begun
   uint32_t report_delay_ms = 0;
   std::atomic<int> late{0}; // reports still to come
 } f;
@@ -36,10 +37,10 @@ bool inside(const std::map<const char *, size_t> &blocks, const void *p) {
   return it != blocks.begin() && static_cast<const char *>(p) < (--it)->first + it->second;
 }
 
-hipError_t launch(const char *name, uint64_t size = 0) {
+hipError_t launch(const char *name, uint64_t pool = 0) {
   std::lock_guard<std::mutex> l(f.m);
   f.launches[name] += 1;
-  f.most[name] = std::max(f.most[name], size);
+  f.pool += pool;
   return f.failing == name ? hipErrorLaunchFailure : hipSuccess;
 }
 } // namespace
@@ -47,8 +48,8 @@ hipError_t launch(const char *name, uint64_t size = 0) {
 extern "C" {
 void fake_reset() {
   std::lock_guard<std::mutex> l(f.m);
-  f.launches.clear(), f.most.clear(), f.reads.clear(), f.failing.clear();
-  f.limit = size_t(1) << 60, f.largest = 0, f.report_delay_ms = 0;
+  f.launches.clear(), f.reads.clear(), f.failing.clear();
+  f.limit = size_t(1) << 60, f.largest = 0, f.pool = 0, f.report_delay_ms = 0;
 }
 void fake_limit(uint64_t bytes) { f.limit = bytes; }
 void fake_fail(const char *name) { f.failing = name; }
@@ -56,7 +57,7 @@ void fake_report_delay(uint32_t ms) { f.report_delay_ms = ms; }
 uint64_t fake_live() { return f.live; }
 uint64_t fake_largest() { return f.largest; }
 uint64_t fake_launches(const char *name) { return f.launches[name]; }
-uint64_t fake_most(const char *name) { return f.most[name]; }
+uint64_t fake_pool() { return f.pool; }
 uint64_t fake_in_flight() {
   uint64_t n = 0;
   for (auto &s : f.reads)
@@ -168,7 +169,7 @@ int noalloc_init(int, std::string *) { return PT_OK; }
 
 namespace gpu {
 hipError_t launch_wf_shade(const WfParams &p, WfKind, hipStream_t) {
-  return launch("wf_shade", p.n_slots);
+  return launch("wf_shade", p.fresh ? p.n_slots : 0);
 }
 hipError_t launch_wf_trace(const WfParams &p, WfKind, uint32_t, hipStream_t) {
   WfReport *rep = p.report;
@@ -196,15 +197,15 @@ hipError_t launch_wf_reduce(const float *, const WorkDivision &, uint32_t, float
   return launch("wf_reduce");
 }
 hipError_t launch_wf_reduce_batch(const float *, const WfReduceItem *, uint32_t, uint32_t,
-                                  uint32_t blocks, uint32_t, float *, hipStream_t) {
-  return launch("wf_reduce_batch", blocks);
+                                  uint32_t, uint32_t, float *, hipStream_t) {
+  return launch("wf_reduce_batch");
 }
-hipError_t launch_megakernel(const MegaParams &, uint32_t a, uint32_t b, bool, hipStream_t) {
-  return launch("mega", b - a);
+hipError_t launch_megakernel(const MegaParams &, uint32_t, uint32_t, bool, hipStream_t) {
+  return launch("mega");
 }
-hipError_t launch_megakernel_batch(const MegaBatchParams &, uint32_t, uint32_t total, uint32_t,
+hipError_t launch_megakernel_batch(const MegaBatchParams &, uint32_t, uint32_t, uint32_t,
                                    hipStream_t) {
-  return launch("mega_batch", total);
+  return launch("mega_batch");
 }
 hipError_t launch_reduce_sample_blocks(const float *, uint32_t, uint32_t, uint32_t, float *,
                                        hipStream_t) {

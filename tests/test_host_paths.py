@@ -36,7 +36,7 @@ def host_library(tmp_path_factory):
     for name, (res, args) in L.SIGNATURES.items():
         if hasattr(lib, name):
             getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
-    for name in ("live", "largest", "launches", "most", "in_flight"):
+    for name in ("live", "largest", "launches", "pool", "in_flight"):
         getattr(lib, "fake_" + name).restype = C.c_uint64
     lib.fake_limit.argtypes = [C.c_uint64]
     return lib
@@ -93,3 +93,27 @@ def test_controls_of_the_hand_over(fake, control, wavefront):
     r.render_rays_batch([(scene, _rays(4096), None)], 64, 0, _settings())
     assert (fake.fake_launches(b"mega_batch") == 0) == wavefront
     assert (fake.fake_launches(b"wf_trace") > 0) == wavefront
+
+
+# the image has 1,572,864 samples in 512 blocks, the batch 262,144 in 1,024:
+# a limit that leaves a launch fewer than 2^20 and 2^18 of them, one that keeps
+# the image's pool below its samples, the whole grid, no limit
+@pytest.mark.parametrize("limit,image_paths,rays_paths", [
+    (1, 0, 0), (341, 0, 0), (342, 1050624, 0), (511, 1569792, 0), (1023, 1572864, 0),
+    (1024, 1572864, 262144), (0, 1572864, 262144)])
+def test_hand_over_honours_the_launch_limit(fake, limit, image_paths, rays_paths):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(1100)
+    s = _settings(max_blocks_per_launch_gpu=limit)
+    s.render_work_division.force_target_samples = 1
+    s.render_work_division.forced_target_samples_per_thread = 12
+
+    def check(call, mega, paths):
+        fake.fake_reset()
+        call()
+        assert (fake.fake_launches(mega) == 0) == (paths > 0)
+        assert fake.fake_pool() == paths
+    check(lambda: r.render(scene, FTW, 256, 256, 24, s), b"mega", image_paths)
+    s.render_work_division.forced_target_samples_per_thread = 1
+    check(lambda: r.render_rays_batch([(scene, _rays(4096), None)], 64, 0, s), b"mega_batch",
+          rays_paths)
