@@ -113,8 +113,8 @@ typedef struct pt_work_division_settings {
 
 /* The integrators give the same image bit for bit. PT_MEGA_KERNEL images of
  * many samples of a mesh (1.6 M of 1,024 triangles and depth 3 or more, 4.2 M of
- * 4,096 triangles with roulette, up to 2^26 samples) run on the Streaming
- * integrator's kernels, which are faster there, and so do ray batches
+ * 4,096 triangles with roulette, up to 2^26 samples), a few of whose paths show
+ * that most go on for some vertices, run on the Streaming integrator's kernels, which are faster there, and so do ray batches
  * (pt_render_rays_batch) of 262,144 samples without steps or with three and
  * more, unless profiling is on, pt_set_megakernel_split is off, or
  * max_blocks_per_launch_gpu leaves a mega-kernel launch few of the samples (2^20

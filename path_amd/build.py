@@ -41,6 +41,7 @@ SOURCES = [
     "host/scene.cpp",
     "host/bvh.cpp",
     "host/settings.cpp",
+    "host/ray_estimate.cpp",
     "host/renderer.cpp",
     "host/streaming.cpp",
     "host/batch.cpp",

@@ -1,5 +1,6 @@
 #include "renderer.h"
 
+#include "ray_estimate.h"
 #include "settings.h"
 
 #include <rocrand/rocrand.h>
@@ -252,27 +253,38 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
 }
 
 // Whether the wavefront renders a MegaKernel image (the same bits: same paths,
-// same sums). It keeps its lanes busy where rays differ in length, but pays two
-// launches an iteration: it wins with many triangles, samples and vertices per
-// path. Mega-kernel / wavefront, us, at depth 1, 4, 7 and Constant 0.25:
+// same sums), of which a launch may take `paths`. It keeps its lanes busy where
+// rays differ in length, but writes and reads each path's state between its
+// vertices and pays two launches an iteration: it wins with many triangles,
+// samples and rays per sample. Mega-kernel / wavefront, us, at depth 1, 4, 7 and
+// Constant 0.25 in a closed room:
 //   356 triangles, 2.1 M samples: 656/798, 1,767/1,417, 2,877/1,912, 2,729/2,339
 //   1,316, 1.0 M: 427/607, 1,138/1,041, 1,775/1,445, 1,903/2,028
 //   5,156, 1.0 M: 505/655, 1,296/1,134, 2,077/1,591, 1,886/2,189
 //   5,156, 4.2 M: 1,575/1,625, 4,504/3,043, 7,408/4,205, 6,440/4,637
 //   20,516, 0.5 M: 492/659, 1,166/1,182, 1,805/1,643, 2,163/2,602
 //   81,956, 4.2 M: 2,446/2,060, 7,650/3,967, 12,806/5,566, 10,717/6,342
-// 36 triangles, 4.2 M samples, depth 4: 1,428/2,091. Depth 3 with 1.6 M samples:
-// 1,497/1,339 (5,156 triangles). Paths without a depth end in a tail of short
-// iterations: with Constant 0.4 and 0.5 the sides meet at 4.2 M samples and
-// 5,156 triangles. Above 2^26 samples their radiances (12 B each) stay out of
-// memory. Launches limited to fewer than 2^20 paths stay with the mega-kernel.
-static bool wavefront_is_faster(const pt_settings &s, uint64_t samples, uint64_t paths,
-                                uint32_t n_tris) {
+// 36 triangles, 4.2 M samples, depth 4: 1,428/2,091. Above 2^26 samples their
+// radiances (12 B each) stay out of memory. Launches limited to fewer than 2^20
+// paths stay with the mega-kernel.
+static bool wavefront_may_be_faster(const pt_settings &s, uint64_t samples, uint64_t paths,
+                                    uint32_t n_tris) {
   if (samples > (1u << 26) || paths < (1u << 20))
     return false;
   return s.term_prob == PT_TERM_N_ITERS
              ? s.n_iters >= 3 && samples >= (3u << 19) && n_tris >= 1024
              : samples >= (1u << 22) && n_tris >= 4096;
+}
+
+// Rays per sample from which it does, of those images. Where rays miss or paths
+// end early it lost: a lone sphere (1.09 rays per sample, 8.4 M samples) 510/1,200,
+// one that fills the film (2.25, 4.2 M) 1,020/1,422; with walls of the room taken
+// away, 5,156 triangles, 1.6 M samples at depths 3 and 7: 620/712 and 903/975 (2.1
+// and 2.2 rays), 795/821 and 1,198/1,153 (2.9 and 3.3), 938/921 and 1,562/1,374
+// (3.9 and 4.9); 4.2 M samples with Constant 0.7, 0.6 and 0.5: 1,659/1,733 (2.3),
+// 2,085/1,957 (2.6), 2,675/2,359 (2.9). So at least 2.6, and six million rays.
+static float wavefront_rays_per_sample(uint64_t samples) {
+  return std::max(2.6f, 6e6f / float(samples));
 }
 
 int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
@@ -392,8 +404,13 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   const uint64_t paths = wavefront ? 0
                                    : hand_over_paths(samples, wd.total_num_blocks(),
                                                      settings.max_blocks_per_launch_gpu);
-  if (!wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
-      wavefront_is_faster(settings, samples, paths, scene_store.dev.n_tris)) {
+  const bool may_hand_over =
+      !wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
+      wavefront_may_be_faster(settings, samples, paths, scene_store.dev.n_tris);
+  const float line = wavefront_rays_per_sample(samples);
+  // (the estimate takes 2 to 25 us of host time)
+  if (may_hand_over && rays_per_sample(scene, settings, spec.film_to_world, x_dim, y_dim, line) >=
+                           line) {
     HandOver hand_over{paths};
     uint64_t wf_rays = 0;
     rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings, rng, x_dim, y_dim,

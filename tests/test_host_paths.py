@@ -62,13 +62,24 @@ def _settings(**kw):
     return s
 
 
-def _scene(n_tris):
+def _scene(n_tris, walls=6, albedo=0.7):
+    """Small triangles in a box with so many of its walls; the camera is at the
+    origin."""
     from path_amd.renderer import Scene, material
     rng = np.random.default_rng(1)
-    v = rng.uniform(-1, 1, (n_tris, 1, 3)) + rng.uniform(-0.05, 0.05, (n_tris, 3, 3))
+    v = [rng.uniform(-1, 1, (n_tris, 1, 3)) + rng.uniform(-0.05, 0.05, (n_tris, 3, 3))]
+    for w in range(walls):
+        axis, side = w % 3, 1.5 if w >= 3 else -1.5  # the first three meet at a corner
+        q = np.array([(side, a, b) for a, b in ((-1.5, -1.5), (1.5, -1.5), (1.5, 1.5), (-1.5, 1.5))])
+        q = np.roll(q, axis, 1)
+        v += [q[[0, 1, 2]][None], q[[0, 2, 3]][None]]
+    v = np.concatenate(v)
     s = Scene()
-    s.add_mesh(v.reshape(-1, 9).astype(np.float32), np.zeros(n_tris, np.uint32),
-               [material("Diffuse", diffuse=(0.5,) * 3, emission=(1, 1, 1))])
+    mats = np.zeros(len(v), np.uint32)
+    mats[0] = 1
+    s.add_mesh(v.reshape(-1, 9).astype(np.float32), mats,
+               [material("Diffuse", diffuse=(albedo,) * 3),
+                material("Diffuse", diffuse=(albedo,) * 3, emission=(1, 1, 1))])
     return s
 
 
@@ -117,3 +128,20 @@ def test_hand_over_honours_the_launch_limit(fake, limit, image_paths, rays_paths
     s.render_work_division.forced_target_samples_per_thread = 1
     check(lambda: r.render_rays_batch([(scene, _rays(4096), None)], 64, 0, s), b"mega_batch",
           rays_paths)
+
+
+# images above the hand-over's sizes whose paths go on, or end at once: rays
+# that miss, dark surfaces and likely termination with roulette
+@pytest.mark.parametrize("tris,walls,albedo,spp,settings,wavefront", [
+    (1100, 6, 0.7, 24, {}, True), (1100, 6, 0.1, 24, {}, True),
+    (1100, 0, 0.7, 24, {}, False), (1100, 0, 0.7, 500, {}, False), (1100, 1, 0.7, 24, {}, False),
+    (4200, 6, 0.7, 64, dict(term_prob="Constant", constant_prob=0.3), True),
+    (4200, 6, 0.7, 64, dict(term_prob="Constant", constant_prob=0.9), False),
+    (4200, 6, 0.7, 64, dict(term_prob="MultiplierFunc"), True),
+    (4200, 6, 0.05, 64, dict(term_prob="MultiplierFunc"), False)])
+def test_images_of_short_paths_stay_on_the_megakernel(fake, tris, walls, albedo, spp, settings,
+                                                      wavefront):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(tris, walls, albedo)
+    r.render(scene, FTW, 256, 256, spp, _settings(**settings))
+    assert (fake.fake_launches(b"mega") == 0) == wavefront
