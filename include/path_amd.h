@@ -117,9 +117,9 @@ typedef struct pt_work_division_settings {
  * that most go on for some vertices, run on the Streaming integrator's kernels, which are faster there, and so do ray batches
  * (pt_render_rays_batch) of 262,144 samples without steps or with three and
  * more, unless profiling is on, pt_set_megakernel_split is off, or
- * max_blocks_per_launch_gpu leaves a mega-kernel launch few of the samples (2^20
- * of an image, 2^18 of a batch); above that, no launch there takes more paths
- * than one of the mega-kernel would. */
+ * max_blocks_per_launch_gpu is too small for that (below 1,366 blocks, or below
+ * the traversal's grid; above, none of its launches that trace or shade has
+ * more blocks either). */
 enum pt_kernel_approach { PT_MEGA_KERNEL = 0, PT_STREAMING = 1 };
 enum pt_accel_type {
   PT_ACCEL_LOOP_ALL = 0,

@@ -676,8 +676,8 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
   return PT_OK;
 }
 
-// The wavefront traces a batch's rays from this many samples on (and, where
-// launches are limited, this many in each), and of three steps or more: the
+// The wavefront traces a batch's rays from this many samples on (and a pool of as
+// many paths, where launches are limited), and of three steps or more: the
 // mega-kernel's waves wait for their longest path, the wavefront pays two
 // launches an iteration. Whole calls, us, mega-kernel /
 // wavefront, six steps: 89,600 samples 1,102 / 1,015, 192,000: 1,292 / 1,356,
@@ -890,7 +890,7 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   // (the stream is synchronised before the staging buffer is used again)
   const size_t sample_floats = size_t(n_img) * total * 3;
   HandOver hand_over{
-      hand_over_paths(total, block_begin[m], settings.max_blocks_per_launch_gpu)};
+      hand_over_paths(r, total, true, settings.max_blocks_per_launch_gpu)};
   if (r.mega_split && !r.profiling && hand_over.max_paths >= kRaysWavefrontMin &&
       (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
     rc = rays_wavefront(r, items, act, desc, mb, settings, rng, with_idx != 0, n_steps, total,

@@ -253,7 +253,7 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
 }
 
 // Whether the wavefront renders a MegaKernel image (the same bits: same paths,
-// same sums), of which a launch may take `paths`. It keeps its lanes busy where
+// same sums) with a pool of `paths`. It keeps its lanes busy where
 // rays differ in length, but writes and reads each path's state between its
 // vertices and pays two launches an iteration: it wins with many triangles,
 // samples and rays per sample. Mega-kernel / wavefront, us, at depth 1, 4, 7 and
@@ -265,8 +265,8 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
 //   20,516, 0.5 M: 492/659, 1,166/1,182, 1,805/1,643, 2,163/2,602
 //   81,956, 4.2 M: 2,446/2,060, 7,650/3,967, 12,806/5,566, 10,717/6,342
 // 36 triangles, 4.2 M samples, depth 4: 1,428/2,091. Above 2^26 samples their
-// radiances (12 B each) stay out of memory. Launches limited to fewer than 2^20
-// paths stay with the mega-kernel.
+// radiances (12 B each) stay out of memory. Pools limited to fewer than 2^20
+// paths (max_blocks_per_launch_gpu) leave the image to the mega-kernel.
 static bool wavefront_may_be_faster(const pt_settings &s, uint64_t samples, uint64_t paths,
                                     uint32_t n_tris) {
   if (samples > (1u << 26) || paths < (1u << 20))
@@ -392,18 +392,9 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   HIP_TRY(hipEventRecord(ev_start, stream));
   const float *final_rgb = nullptr;
   bool wavefront = settings.kernel_approach == PT_STREAMING;
-  WorkDivision wd;
-  if (!wavefront) {
-    if (!WorkDivision::make(work_division_settings(settings.render_work_division),
-                            samples_per, x_dim, y_dim, &wd))
-      return set_error(PT_ERR_INVALID, "invalid render work division settings");
-    if (wd.block_size > 1024)
-      return set_error(PT_ERR_INVALID, "block_size above 1024");
-  }
   const uint64_t samples = uint64_t(n_pixels) * samples_per;
-  const uint64_t paths = wavefront ? 0
-                                   : hand_over_paths(samples, wd.total_num_blocks(),
-                                                     settings.max_blocks_per_launch_gpu);
+  const uint64_t paths =
+      hand_over_paths(*this, samples, false, settings.max_blocks_per_launch_gpu);
   const bool may_hand_over =
       !wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
       wavefront_may_be_faster(settings, samples, paths, scene_store.dev.n_tris);
@@ -426,6 +417,12 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
       return rc;
   }
   if (!wavefront) {
+    WorkDivision wd;
+    if (!WorkDivision::make(work_division_settings(settings.render_work_division),
+                            samples_per, x_dim, y_dim, &wd))
+      return set_error(PT_ERR_INVALID, "invalid render work division settings");
+    if (wd.block_size > 1024)
+      return set_error(PT_ERR_INVALID, "block_size above 1024");
     const size_t image_floats = size_t(wd.num_sample_blocks) * n_pixels * 3;
     HIP_TRY(rgb.ensure(image_floats * (per_step ? out.n_steps : 1)));
     gpu::MegaParams p{};

@@ -10,7 +10,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <memory>
 #include <string>
 
@@ -340,16 +339,11 @@ struct HandOver {
   uint64_t max_paths;
   bool no_memory = false;
 };
-// Paths of the pool of work handed over: at most kHandOverPool, and at most the
-// samples that a mega-kernel launch of max_blocks (0: all) of its grid's blocks
-// has, so that a limit on launches keeps bounding them (each of the wavefront's
-// takes its paths one vertex further).
-constexpr uint64_t kHandOverPool = 1u << 22;
-inline uint64_t hand_over_paths(uint64_t samples, uint64_t blocks, uint32_t max_blocks) {
-  if (max_blocks != 0 && max_blocks < blocks)
-    samples = uint64_t(double(samples) / double(blocks) * max_blocks);
-  return std::min(samples, kHandOverPool);
-}
+// Paths of the pool of work handed over: at most 2^22, and so few that no launch
+// that traces or shades has more than max_blocks blocks (0: any number), since
+// the caller has limited the mega-kernel's launches to that; 0 if that cannot be.
+uint64_t hand_over_paths(const pt_renderer &r, uint64_t samples, bool batched,
+                         uint32_t max_blocks);
 int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
                      const gpu::DeviceScene &scene, uint32_t samples_per,
                      const pt_settings &settings, const gpu::RngParams &rng,

@@ -49,6 +49,30 @@ static size_t counter_words(int n) {
   return gpu::kGroupStride + size_t(n) * gpu::kGroupCounterWords;
 }
 
+// Pipelines of a pool of n_slots paths: a given number is kept to one shade
+// block each.
+static uint32_t pipelines(const pt_renderer &r, uint32_t n_slots) {
+  const uint32_t n = r.n_pipes ? std::min(r.n_pipes, n_slots / 256)
+                               : std::min(3u, n_slots / kMinPipeSlots);
+  return std::max(1u, std::min(n, uint32_t(kMaxPipes)));
+}
+
+uint64_t hand_over_paths(const pt_renderer &r, uint64_t samples, bool batched,
+                         uint32_t max_blocks) {
+  uint64_t paths = std::min<uint64_t>(samples, 1u << 22);
+  if (max_blocks == 0)
+    return paths;
+  if (max_blocks < uint32_t(r.n_cus) * r.trace_blocks_for(batched))
+    return 0; // (the traversal's grid, whatever the pool)
+  // 256 paths per shade block; a smaller pool may have fewer pipelines
+  for (;;) {
+    const uint64_t most = uint64_t(max_blocks) * 256 * pipelines(r, uint32_t(paths));
+    if (paths <= most)
+      return paths;
+    paths = most;
+  }
+}
+
 int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
                     uint32_t n_slots, uint64_t total_samples, gpu::WfKind kind,
                     uint32_t trace_blocks) {
@@ -69,10 +93,7 @@ int wavefront_alloc(pt_renderer &r, WfPipes &w, const gpu::WfParams &base,
   // Pipelines have an equal share of the slots each, their own stream, queues
   // and counters: the memory-bound shade step of one overlaps the ALU-bound
   // traversal of another.
-  // A given number of pipelines is kept to one shade block each.
-  const uint32_t pipes = r.n_pipes ? std::min(r.n_pipes, n_slots / 256)
-                                   : std::min(3u, n_slots / kMinPipeSlots);
-  w.n = int(std::max(1u, std::min(pipes, uint32_t(kMaxPipes))));
+  w.n = int(pipelines(r, n_slots));
   uint32_t first[kMaxPipes + 1] = {0};
   for (int h = 0; h < w.n; ++h) {
     const uint32_t left = n_slots - first[h], pipes_left = uint32_t(w.n - h);

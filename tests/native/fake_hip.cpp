@@ -27,7 +27,8 @@ struct Fake {
   std::map<hipStream_t, int> reads;               // copies out of pinned memory
   std::string failing;
   size_t limit = size_t(1) << 60, live = 0, largest = 0;
-  uint64_t pool = 0; // paths of the wavefront renders begun
+  uint64_t pool = 0;   // paths of the wavefront renders begun
+  uint64_t blocks = 0; // largest grid of a wavefront launch
   uint32_t report_delay_ms = 0;
   std::atomic<int> late{0}; // reports still to come
 } f;
@@ -37,10 +38,11 @@ bool inside(const std::map<const char *, size_t> &blocks, const void *p) {
   return it != blocks.begin() && static_cast<const char *>(p) < (--it)->first + it->second;
 }
 
-hipError_t launch(const char *name, uint64_t pool = 0) {
+hipError_t launch(const char *name, uint64_t pool = 0, uint64_t blocks = 0) {
   std::lock_guard<std::mutex> l(f.m);
   f.launches[name] += 1;
   f.pool += pool;
+  f.blocks = std::max(f.blocks, blocks);
   return f.failing == name ? hipErrorLaunchFailure : hipSuccess;
 }
 } // namespace
@@ -49,7 +51,7 @@ extern "C" {
 void fake_reset() {
   std::lock_guard<std::mutex> l(f.m);
   f.launches.clear(), f.reads.clear(), f.failing.clear();
-  f.limit = size_t(1) << 60, f.largest = 0, f.pool = 0, f.report_delay_ms = 0;
+  f.limit = size_t(1) << 60, f.largest = 0, f.pool = f.blocks = 0, f.report_delay_ms = 0;
 }
 void fake_limit(uint64_t bytes) { f.limit = bytes; }
 void fake_fail(const char *name) { f.failing = name; }
@@ -58,6 +60,7 @@ uint64_t fake_live() { return f.live; }
 uint64_t fake_largest() { return f.largest; }
 uint64_t fake_launches(const char *name) { return f.launches[name]; }
 uint64_t fake_pool() { return f.pool; }
+uint64_t fake_blocks() { return f.blocks; }
 uint64_t fake_in_flight() {
   uint64_t n = 0;
   for (auto &s : f.reads)
@@ -169,9 +172,9 @@ int noalloc_init(int, std::string *) { return PT_OK; }
 
 namespace gpu {
 hipError_t launch_wf_shade(const WfParams &p, WfKind, hipStream_t) {
-  return launch("wf_shade", p.fresh ? p.n_slots : 0);
+  return launch("wf_shade", p.fresh ? p.n_slots : 0, p.n_shade_blocks);
 }
-hipError_t launch_wf_trace(const WfParams &p, WfKind, uint32_t, hipStream_t) {
+hipError_t launch_wf_trace(const WfParams &p, WfKind, uint32_t blocks, hipStream_t) {
   WfReport *rep = p.report;
   const uint32_t it = ++p.counters[kIterations];
   auto tell = [rep, it] {
@@ -188,7 +191,7 @@ hipError_t launch_wf_trace(const WfParams &p, WfKind, uint32_t, hipStream_t) {
   } else {
     tell();
   }
-  return launch("wf_trace");
+  return launch("wf_trace", 0, blocks);
 }
 hipError_t launch_wf_finish(const WfParams &, WfKind, uint32_t, hipStream_t) {
   return launch("wf_finish");

@@ -36,7 +36,7 @@ def host_library(tmp_path_factory):
     for name, (res, args) in L.SIGNATURES.items():
         if hasattr(lib, name):
             getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
-    for name in ("live", "largest", "launches", "pool", "in_flight"):
+    for name in ("live", "largest", "launches", "pool", "blocks", "in_flight"):
         getattr(lib, "fake_" + name).restype = C.c_uint64
     lib.fake_limit.argtypes = [C.c_uint64]
     return lib
@@ -106,27 +106,27 @@ def test_controls_of_the_hand_over(fake, control, wavefront):
     assert (fake.fake_launches(b"wf_trace") > 0) == wavefront
 
 
-# the image has 1,572,864 samples in 512 blocks, the batch 262,144 in 1,024:
-# a limit that leaves a launch fewer than 2^20 and 2^18 of them, one that keeps
-# the image's pool below its samples, the whole grid, no limit
+# 6,291,456 samples each; the traversal's grid is 3 blocks per CU for an image
+# and 6 for a batch. 3 x 256 paths per block of the limit; an image's pool of
+# fewer than 2^20 is not worth it
 @pytest.mark.parametrize("limit,image_paths,rays_paths", [
-    (1, 0, 0), (341, 0, 0), (342, 1050624, 0), (511, 1569792, 0), (1023, 1572864, 0),
-    (1024, 1572864, 262144), (0, 1572864, 262144)])
+    (0, 1 << 22, 1 << 22), (1 << 20, 1 << 22, 1 << 22), (5462, 1 << 22, 1 << 22),
+    (4096, 3145728, 3145728), (1536, 1179648, 1179648), (1535, 1178880, 0), (1366, 1049088, 0),
+    (1365, 0, 0), (767, 0, 0), (1, 0, 0)])
 def test_hand_over_honours_the_launch_limit(fake, limit, image_paths, rays_paths):
     from path_amd.renderer import Renderer
     r, scene = Renderer(0), _scene(1100)
     s = _settings(max_blocks_per_launch_gpu=limit)
-    s.render_work_division.force_target_samples = 1
-    s.render_work_division.forced_target_samples_per_thread = 12
 
     def check(call, mega, paths):
         fake.fake_reset()
         call()
         assert (fake.fake_launches(mega) == 0) == (paths > 0)
         assert fake.fake_pool() == paths
-    check(lambda: r.render(scene, FTW, 256, 256, 24, s), b"mega", image_paths)
-    s.render_work_division.forced_target_samples_per_thread = 1
-    check(lambda: r.render_rays_batch([(scene, _rays(4096), None)], 64, 0, s), b"mega_batch",
+        if paths and limit:
+            assert fake.fake_blocks() <= limit
+    check(lambda: r.render(scene, FTW, 512, 256, 48, s), b"mega", image_paths)
+    check(lambda: r.render_rays_batch([(scene, _rays(32768), None)], 192, 0, s), b"mega_batch",
           rays_paths)
 
 
