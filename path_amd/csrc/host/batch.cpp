@@ -687,6 +687,11 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
 // many bytes.
 constexpr uint64_t kRaysWavefrontMin = 1u << 18;
 constexpr size_t kRaysWavefrontBytes = size_t(4) << 30;
+// And it has to have this many samples for each image (item and step) that is
+// reduced by launches of its own, two where the mega-kernel has one, ms: 200
+// items x 10 rays x 256 samples, six steps, 5.19 / 10.07; 48 x 9 x 4,096: 3.86 /
+// 4.12; 48 x 9 x 20,000: 12.4 / 11.2; 400 x 2 x 20,000, eight steps: 50.4 / 52.7.
+constexpr uint64_t kRaysPerReduction = 1u << 14;
 
 // The wavefront's part of render_rays_batch: scenes, rays and indices are on the
 // device. Values are summed like the mega-kernel's, so they are the same bits.
@@ -694,7 +699,7 @@ constexpr size_t kRaysWavefrontBytes = size_t(4) << 30;
 static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
                           const std::vector<uint32_t> &act,
                           const std::vector<gpu::SceneDesc> &desc,
-                          const std::vector<gpu::MegaBatchItem> &mb, const pt_settings &settings,
+                          const BatchReduction &red, const pt_settings &settings,
                           const gpu::RngParams &rng, bool with_idx, uint32_t n_steps,
                           uint64_t total, uint64_t n_rays,
                           std::chrono::steady_clock::time_point t0, double *seconds,
@@ -725,9 +730,6 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
     hand_over->no_memory = true;
     return PT_OK;
   }
-  BatchReduction red;
-  for (uint32_t j = 0; j < m; ++j)
-    red.add(mb[j].wd, desc[j].pixel_off);
   if ((rc = red.upload(r)) != PT_OK)
     return rc;
   HIP_TRY(hipEventRecord(r.ev_start, s));
@@ -891,9 +893,13 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   const size_t sample_floats = size_t(n_img) * total * 3;
   HandOver hand_over{
       hand_over_paths(r, total, true, settings.max_blocks_per_launch_gpu)};
+  BatchReduction red;
+  for (uint32_t j = 0; j < m; ++j)
+    red.add(mb[j].wd, desc[j].pixel_off);
   if (r.mega_split && !r.profiling && hand_over.max_paths >= kRaysWavefrontMin &&
-      (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes) {
-    rc = rays_wavefront(r, items, act, desc, mb, settings, rng, with_idx != 0, n_steps, total,
+      (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes &&
+      total >= red.alone.size() * n_img * kRaysPerReduction) {
+    rc = rays_wavefront(r, items, act, desc, red, settings, rng, with_idx != 0, n_steps, total,
                         ray_total, t0, seconds, &hand_over);
     if (!hand_over.no_memory)
       return rc;

@@ -145,3 +145,19 @@ def test_images_of_short_paths_stay_on_the_megakernel(fake, tris, walls, albedo,
     r, scene = Renderer(0), _scene(tris, walls, albedo)
     r.render(scene, FTW, 256, 256, spp, _settings(**settings))
     assert (fake.fake_launches(b"mega") == 0) == wavefront
+
+
+# items whose rays have several sample blocks are reduced one by one: 16,384
+# samples for each such image, or the mega-kernel
+@pytest.mark.parametrize("items,rays,spp,steps,wavefront", [
+    (200, 10, 256, 6, False), (1, 2000, 256, 6, True), (31, 4, 3000, 3, False), (7, 4, 20000, 3, True),
+    (200, 200, 16, 6, True)])
+def test_ray_batches_of_many_reductions(fake, items, rays, spp, steps, wavefront):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(20)
+    s = _settings()
+    s.render_work_division.max_samples_per_thread = 8
+    out = r.render_rays_batch([(scene, _rays(rays), None)] * items, spp, steps, s)
+    assert len(out) == items
+    assert (fake.fake_launches(b"mega_batch") == 0) == wavefront
+    assert fake.fake_launches(b"wf_reduce") <= items * rays * spp >> 14
