@@ -875,7 +875,7 @@ def main(argv=None):
     ap.add_argument("--overlap-threshold", type=float, default=0.0,
                     help="with --spatial-splits: overlap_threshold (default 1e-5)")
     ap.add_argument("--pipelines", type=int, default=0,
-                    help="wavefront pipelines per render (default 3)")
+                    help="wavefront pipelines per render (0: three, fewer for small pools)")
     ap.add_argument("--mlp-forward", action="store_true",
                     help="only time the radiance MLP's fused inference forward (2^20 queries, "
                          "--steps launches)")

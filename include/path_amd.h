@@ -398,7 +398,7 @@ int pt_set_launch_params(pt_renderer *r, uint32_t trace_blocks_per_cu,
 enum { PT_BVH_HOST_SAH = 0, PT_BVH_GPU_LBVH = 1, PT_BVH_GPU_PLOC = 2 };
 /* Independent wavefront pipelines a Streaming render splits its path pool
  * into (1..4; each at least 256 paths), each on its own stream and host thread.
- * Without this call: three, fewer for pools below 3 x 2^18 paths. Results never
+ * 0, the default: three, fewer for pools below 3 x 2^18 paths. Results never
  * depend on it. */
 int pt_set_pipelines(pt_renderer *r, uint32_t n);
 /* MegaKernel launch shape (no reference counterpart; the reference runs one

@@ -553,8 +553,9 @@ int pt_set_launch_params(pt_renderer *r, uint32_t trace_blocks_per_cu,
 }
 
 int pt_set_pipelines(pt_renderer *r, uint32_t n) {
-  if (!r || n == 0 || n > uint32_t(kMaxPipes))
-    return fail(PT_ERR_INVALID, "pipelines must be in [1, " + std::to_string(kMaxPipes) + "]");
+  if (!r || n > uint32_t(kMaxPipes))
+    return fail(PT_ERR_INVALID, "pipelines must be in [1, " + std::to_string(kMaxPipes) +
+                                     "], or 0 for the default");
   r->n_pipes = n;
   return PT_OK;
 }

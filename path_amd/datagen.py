@@ -133,8 +133,8 @@ def set_launch_params(renderer: Renderer, trace_blocks_per_cu: int = 0,
 
 
 def set_pipelines(renderer: Renderer, n: int) -> None:
-    """Wavefront pipelines of a Streaming render (1-4; unless set, three,
-    fewer for small path pools)."""
+    """Wavefront pipelines of a Streaming render: 1-4, or 0 (the default) for
+    three, fewer for small path pools."""
     L.check(L.lib().pt_set_pipelines(renderer.handle, n))
 
 

@@ -121,8 +121,7 @@ def test_streaming_image_equals_megakernel(renderer, request, which, spp, size):
     s = _settings("Streaming")
     wf, _ = renderer.render(scene, ftw, size, size, spp, s)
     assert np.array_equal(mk.view(np.uint32), wf.view(np.uint32))
-    # small path pools force many regenerations per slot; below 512 slots the
-    # pool runs as one pipeline instead of two
+    # small path pools force many regenerations per slot
     for pool in (1000, 300):
         s.max_num_samples_per_launch = pool
         wf2, _ = renderer.render(scene, ftw, size, size, spp, s)
@@ -136,7 +135,7 @@ def test_streaming_image_equals_megakernel(renderer, request, which, spp, size):
             wf3, _ = renderer.render(scene, ftw, size, size, spp, s)
             assert np.array_equal(mk.view(np.uint32), wf3.view(np.uint32)), n
     finally:
-        set_pipelines(renderer, 3)
+        set_pipelines(renderer, 0)
 
 
 @pytest.mark.parametrize("which", ["cornell_sphere", "benchmark_scene"])

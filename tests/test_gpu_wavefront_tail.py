@@ -44,10 +44,12 @@ def test_streaming_equals_megakernel(renderer, request, which, term, rng, x, y, 
             img, _ = renderer.render(scene, ftw, x, y, spp, s)
             assert np.array_equal(img.view(np.uint32), mega.view(np.uint32)), (iters, graphs)
             assert renderer.last_stats().rays == rays, (iters, graphs)
+            auto = min(3, max(1, x * y * spp >> 18))
+            assert renderer.last_stats().pipelines == (pipes or auto)
     finally:
         set_launch_params(renderer, 0, 1, False)
         if pipes:
-            set_pipelines(renderer, 3)
+            set_pipelines(renderer, 0)
 
 
 # 1 and 3 samples: finished after the first iteration; 40: after several.

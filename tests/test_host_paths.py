@@ -161,3 +161,17 @@ def test_ray_batches_of_many_reductions(fake, items, rays, spp, steps, wavefront
     assert len(out) == items
     assert (fake.fake_launches(b"mega_batch") == 0) == wavefront
     assert fake.fake_launches(b"wf_reduce") <= items * rays * spp >> 14
+
+
+def test_pipelines_back_to_the_default(fake):
+    from path_amd.datagen import set_pipelines
+    from path_amd.renderer import Renderer
+    r, scene, s = Renderer(0), _scene(20), _settings(kernel_approach="Streaming")
+    for set_to, small, large in ((None, 1, 3), (4, 4, 4), (1, 1, 1), (0, 1, 3)):
+        if set_to is not None:
+            set_pipelines(r, set_to)
+        for spp, n in ((16, small), (200, large)):
+            r.render(scene, FTW, 64, 64, spp, s)
+            assert r.last_stats().pipelines == n
+    with pytest.raises(L.PathError):
+        set_pipelines(r, 5)
