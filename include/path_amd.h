@@ -119,7 +119,9 @@ typedef struct pt_work_division_settings {
  * more, unless profiling is on, pt_set_megakernel_split is off, or
  * max_blocks_per_launch_gpu is too small for that (below 1,366 blocks, or below
  * the traversal's grid; above, none of its launches that trace or shade has
- * more blocks either). */
+ * more blocks either). Those take device memory for the paths and their
+ * values; where it does not fit, the mega-kernel runs. The renderer keeps about
+ * a gigabyte of it. */
 enum pt_kernel_approach { PT_MEGA_KERNEL = 0, PT_STREAMING = 1 };
 enum pt_accel_type {
   PT_ACCEL_LOOP_ALL = 0,

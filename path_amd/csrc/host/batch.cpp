@@ -492,7 +492,14 @@ struct BatchReduction {
       alone.push_back({wd, 0, pixel_off});
     }
   }
-  int upload(pt_renderer &r) const {
+  // Allocates what run() needs and uploads the items.
+  int prepare(pt_renderer &r) const {
+    size_t most = 0;
+    for (const gpu::WfReduceItem &it : alone)
+      if (it.wd.num_sample_blocks != 1)
+        most = std::max(most, size_t(it.wd.x_dim) * it.wd.y_dim * 3 * it.wd.num_sample_blocks);
+    if (most)
+      HIP_TRY(r.rgb2.ensure(most));
     HIP_TRY(r.b_reduce.upload(together.data(), together.size(), r.stream));
     return PT_OK;
   }
@@ -502,15 +509,15 @@ struct BatchReduction {
       HIP_TRY(gpu::launch_wf_reduce_batch(samples, r.b_reduce.ptr, uint32_t(together.size()),
                                           together[0].wd.block_size, blocks, spp, out, s));
     for (const gpu::WfReduceItem &it : alone) {
-      const size_t off = it.pixel_off, px = size_t(it.wd.x_dim) * it.wd.y_dim;
+      const size_t off = it.pixel_off;
+      const uint32_t px = it.wd.x_dim * it.wd.y_dim;
       if (it.wd.num_sample_blocks == 1) {
         HIP_TRY(gpu::launch_wf_reduce(samples + 3 * off * spp, it.wd, spp, out + 3 * off, s));
         continue;
       }
-      HIP_TRY(r.rgb2.ensure(px * 3 * it.wd.num_sample_blocks));
       HIP_TRY(gpu::launch_wf_reduce(samples + 3 * off * spp, it.wd, spp, r.rgb2.ptr, s));
-      HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, it.wd.num_sample_blocks, uint32_t(px),
-                                               spp, out + 3 * off, s));
+      HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb2.ptr, it.wd.num_sample_blocks, px, spp,
+                                               out + 3 * off, s));
     }
     return PT_OK;
   }
@@ -609,7 +616,7 @@ int render_batch(pt_renderer &r, const pt_batch_item *items, uint32_t n,
       return set_error(PT_ERR_INVALID, "invalid render work division settings");
     red.add(wd, desc[i].pixel_off);
   }
-  if ((rc = red.upload(r)) != PT_OK)
+  if ((rc = red.prepare(r)) != PT_OK)
     return rc;
   r.stats = pt_render_stats{};
   r.stats.profiled = r.profiling ? 1u : 0u;
@@ -706,12 +713,9 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
                           HandOver *hand_over) {
   hipStream_t s = r.stream;
   const uint32_t n_img = n_steps ? n_steps : 1, m = uint32_t(act.size());
-  if (r.ray_samples.ensure(size_t(n_img) * total * 3) != hipSuccess) {
-    (void)hipGetLastError();
-    hand_over->no_memory = true;
-    return PT_OK;
-  }
-  HIP_TRY(r.rgb.ensure(size_t(n_img) * n_rays * 3));
+  if (r.ray_samples.ensure(size_t(n_img) * total * 3) != hipSuccess ||
+      r.rgb.ensure(size_t(n_img) * n_rays * 3) != hipSuccess)
+    return hand_over->does_not_fit(r);
   gpu::WfParams p{};
   p.settings = integrator_settings(settings);
   p.rng = rng;
@@ -725,13 +729,8 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
   const uint32_t trace_blocks = uint32_t(r.n_cus) * r.trace_blocks_for(true);
   WfPipes w;
   int rc = wavefront_alloc(r, w, p, uint32_t(slots), total, gpu::kWfRays, trace_blocks);
-  if (rc != PT_OK) {
-    (void)hipGetLastError();
-    hand_over->no_memory = true;
-    return PT_OK;
-  }
-  if ((rc = red.upload(r)) != PT_OK)
-    return rc;
+  if (rc != PT_OK || red.prepare(r) != PT_OK)
+    return hand_over->does_not_fit(r);
   HIP_TRY(hipEventRecord(r.ev_start, s));
   if (n_steps) // steps that a path does not reach stay zero
     HIP_TRY(hipMemsetAsync(r.ray_samples.ptr, 0, size_t(n_img) * total * 3 * sizeof(float), s));
@@ -759,6 +758,7 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
   // given first hits went through the queues untraced
   r.stats.rays = r.stats.ext_rays + r.stats.shadow_rays - (with_idx ? total : 0);
   r.stats.samples = total;
+  HandOver::trim(r);
   if (seconds)
     *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return PT_OK;

@@ -399,6 +399,8 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
       !wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
       wavefront_may_be_faster(settings, samples, paths, scene_store.dev.n_tris);
   const float line = wavefront_rays_per_sample(samples);
+  if (out.type == PT_OUTPUT_BGRA) // (before the wavefront's buffers)
+    HIP_TRY(bgra.ensure(n_pixels));
   // (the estimate takes 2 to 25 us of host time)
   if (may_hand_over && rays_per_sample(scene, settings, spec.film_to_world, x_dim, y_dim, line) >=
                            line) {
@@ -464,10 +466,8 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
       final_rgb = rgb2.ptr;
     }
   }
-  if (out.type == PT_OUTPUT_BGRA) {
-    HIP_TRY(bgra.ensure(n_pixels));
+  if (out.type == PT_OUTPUT_BGRA)
     HIP_TRY(gpu::launch_to_bgra(final_rgb, n_pixels, bgra.ptr, stream));
-  }
   HIP_TRY(hipEventRecord(ev_stop, stream));
   // Host outputs go through pinned staging (one DMA copy, then a host
   // memcpy): copying straight into pageable memory took as long as a small
@@ -504,7 +504,9 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   stats.rays = wavefront
                    ? stats.ext_rays + stats.shadow_rays
                    : rays_traced;
-  stats.samples = uint64_t(samples_per) * n_pixels;
+  stats.samples = samples;
+  if (wavefront && settings.kernel_approach == PT_MEGA_KERNEL)
+    HandOver::trim(*this);
   double secs = std::chrono::duration<double>(t1 - t0).count();
   if (seconds)
     *seconds = secs;

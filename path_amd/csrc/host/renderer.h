@@ -100,21 +100,21 @@ template <class T> struct DeviceBuf {
   DeviceBuf() = default;
   DeviceBuf(const DeviceBuf &) = delete;
   DeviceBuf &operator=(const DeviceBuf &) = delete;
-  ~DeviceBuf() {
-    if (ptr)
-      (void)hipFree(ptr);
-  }
+  ~DeviceBuf() { release(); }
   hipError_t ensure(size_t n) {
     if (n <= count && ptr)
       return hipSuccess;
-    if (ptr)
-      (void)hipFree(ptr);
-    ptr = nullptr;
-    count = 0;
+    release();
     hipError_t e = hipMalloc(&ptr, (n ? n : 1) * sizeof(T));
     if (e == hipSuccess)
       count = n;
     return e;
+  }
+  void release() {
+    if (ptr)
+      (void)hipFree(ptr);
+    ptr = nullptr;
+    count = 0;
   }
   hipError_t upload(const T *src, size_t n, hipStream_t s) {
     hipError_t e = ensure(n);
@@ -338,6 +338,14 @@ int render_adjoint(pt_renderer &r, const pt_scene &scene, const float film_to_wo
 struct HandOver {
   uint64_t max_paths;
   bool no_memory = false;
+  // Gives back what the wavefront holds (but the last Streaming render's
+  // samples), so that the mega-kernel finds the room it would have had.
+  int does_not_fit(pt_renderer &r);
+  // After a render: per-sample values above kKept are given back. (Allocating
+  // and freeing 0.5 to 0.8 GB takes 0.34 ms, 2 to 4 GB 0.65 ms, where the paths
+  // of so many values take more than 20 ms.)
+  static constexpr size_t kKept = size_t(512) << 20;
+  static void trim(pt_renderer &r);
 };
 // Paths of the pool of work handed over: at most 2^22, and so few that no launch
 // that traces or shades has more than max_blocks blocks (0: any number), since

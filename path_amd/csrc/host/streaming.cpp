@@ -57,6 +57,32 @@ static uint32_t pipelines(const pt_renderer &r, uint32_t n_slots) {
   return std::max(1u, std::min(n, uint32_t(kMaxPipes)));
 }
 
+int HandOver::does_not_fit(pt_renderer &r) {
+  (void)hipGetLastError();
+  no_memory = true;
+  r.ray_samples.release();
+  r.wf_meta.release();
+  r.wf_hit_ext.release();
+  r.wf_hit_light.release();
+  r.wf_mult.release();
+  r.wf_light_dir.release();
+  r.wf_light.release();
+  r.wf_total.release();
+  r.wf_origin.release();
+  r.wf_dir.release();
+  r.wf_q_ext.release();
+  r.wf_q_shadow.release();
+  r.wf_stack_overflow.release();
+  r.wf_counters.release();
+  r.wf_scene.release();
+  return PT_OK;
+}
+
+void HandOver::trim(pt_renderer &r) {
+  if (r.ray_samples.count * sizeof(float) > kKept)
+    r.ray_samples.release();
+}
+
 uint64_t hand_over_paths(const pt_renderer &r, uint64_t samples, bool batched,
                          uint32_t max_blocks) {
   uint64_t paths = std::min<uint64_t>(samples, 1u << 22);
@@ -383,23 +409,20 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
   p.x_dim = x_dim;
   p.y_dim = y_dim;
   if (hand_over) {
-    if (r.ray_samples.ensure(size_t(total) * 3) != hipSuccess) {
-      (void)hipGetLastError();
-      hand_over->no_memory = true;
-      return PT_OK;
-    }
+    if (r.ray_samples.ensure(size_t(total) * 3) != hipSuccess)
+      return hand_over->does_not_fit(r);
     p.out_samples = r.ray_samples.ptr;
   }
   WfPipes w;
   int rc = wavefront_alloc(r, w, p, uint32_t(slots64), total, gpu::kWfImage, trace_blocks);
-  if (rc != PT_OK && hand_over) {
-    (void)hipGetLastError();
-    hand_over->no_memory = true;
-    return PT_OK;
-  }
   if (rc != PT_OK)
-    return rc;
-  HIP_TRY(r.rgb.ensure(size_t(wd.num_sample_blocks) * n_pixels * 3));
+    return hand_over ? hand_over->does_not_fit(r) : rc;
+  hipError_t e = r.rgb.ensure(size_t(wd.num_sample_blocks) * n_pixels * 3);
+  if (e == hipSuccess && wd.num_sample_blocks != 1)
+    e = r.rgb2.ensure(size_t(n_pixels) * 3);
+  if (e != hipSuccess && hand_over)
+    return hand_over->does_not_fit(r);
+  HIP_TRY(e);
   rc = wavefront_run(r, w, gpu::kWfImage, trace_blocks, r.iters_per_sync);
   if (rc != PT_OK)
     return rc;
@@ -407,7 +430,6 @@ int render_streaming(pt_renderer &r, const pt_sample_spec &spec,
   HIP_TRY(gpu::launch_wf_reduce(w.p[0].out_samples, wd, samples_per, r.rgb.ptr, s));
   const float *out = r.rgb.ptr;
   if (wd.num_sample_blocks != 1) {
-    HIP_TRY(r.rgb2.ensure(size_t(n_pixels) * 3));
     HIP_TRY(gpu::launch_reduce_sample_blocks(r.rgb.ptr, wd.num_sample_blocks,
                                              uint32_t(n_pixels), samples_per,
                                              r.rgb2.ptr, s));

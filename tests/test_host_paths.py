@@ -175,3 +175,61 @@ def test_pipelines_back_to_the_default(fake):
             assert r.last_stats().pipelines == n
     with pytest.raises(L.PathError):
         set_pipelines(r, 5)
+
+
+def _image_call(r, scene):
+    s = _settings()
+    s.render_work_division.max_samples_per_thread = 1  # two sample blocks
+    r.render(scene, FTW, 96, 64, 600, s, output="BGRA")
+
+
+def _rays_call(r, scene):
+    r.render_rays_batch([(scene, _rays(3000, i), None) for i in range(4)], 100, 8, _settings())
+
+
+# Whatever of the wavefront's memory fits: a call that the mega-kernel alone can
+# do is done, and leaves no more memory taken than the mega-kernel does
+@pytest.mark.parametrize("call,mega", [(_image_call, b"mega"), (_rays_call, b"mega_batch")])
+def test_hand_over_without_memory(fake, call, mega):
+    from path_amd.renderer import Renderer
+    scene = _scene(1100)
+
+    def run(split, room):
+        fake.fake_reset()
+        gc.collect()
+        start = fake.fake_live()
+        fake.fake_limit(start + room)
+        r = Renderer(0)
+        r.set_megakernel_split(split)
+        try:
+            call(r, scene)
+        except L.PathError:
+            return None
+        return fake.fake_live() - start, fake.fake_launches(mega) > 0
+    alone, _ = run(False, 1 << 50)
+    full, on_mega = run(True, 1 << 50)
+    assert not on_mega and full > 2 * alone
+    for room in (*np.linspace(alone, full, 60, endpoint=False).astype(int),
+                 *range(full - 400, full, 40)):
+        got = run(True, int(room))
+        assert got is not None and got[1] and got[0] <= alone, room
+    assert run(True, full) == (full, False)
+    assert run(False, alone - 1) is None
+
+
+# per-sample values of 0.8 GB and 0.6 GB are not kept; 10 MB are
+@pytest.mark.parametrize("call,freed", [
+    (lambda r, s: r.render(s, FTW, 1024, 1024, 64, _settings()), True),
+    (lambda r, s: r.render(s, FTW, 1024, 1024, 2, _settings()), False),
+    (lambda r, s: r.render_rays_batch([(s, _rays(200000), None)], 32, 8, _settings()), True),
+    (lambda r, s: r.render_rays_batch([(s, _rays(9000), None)], 32, 3, _settings()), False)])
+def test_large_values_are_given_back(fake, call, freed):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(1100)
+    call(r, scene)
+    assert fake.fake_launches(b"wf_trace") > 0
+    values = fake.fake_largest()
+    before = fake.fake_live()
+    call(r, scene)
+    assert fake.fake_live() == before
+    assert (values > 512 << 20) == freed and (before < 900 << 20)
