@@ -764,6 +764,17 @@ static int rays_wavefront(pt_renderer &r, const pt_ray_batch_item *items,
   return PT_OK;
 }
 
+// Waits for a stream when a scope ends early, so that the pinned memory its
+// copies read is free again.
+struct WaitUnlessDone {
+  hipStream_t s;
+  bool done = false;
+  ~WaitUnlessDone() {
+    if (!done)
+      (void)hipStreamSynchronize(s);
+  }
+};
+
 int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n,
                       uint32_t spp, uint32_t n_steps, const pt_settings &settings,
                       double *seconds) {
@@ -861,6 +872,9 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
     final_off[j + 1] =
         final_off[j] + (wd.num_sample_blocks == 1 ? 0 : size_t(n_img) * it.n_rays * 3);
   }
+  BatchReduction red; // (of the wavefront)
+  for (uint32_t j = 0; j < m; ++j)
+    red.add(mb[j].wd, desc[j].pixel_off);
   // rays and triangle indices through pinned staging
   const size_t ray_bytes = size_t(ray_total) * 6 * sizeof(float);
   const size_t idx_bytes = with_idx ? size_t(ray_total) * sizeof(uint32_t) : 0;
@@ -874,6 +888,7 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
       std::memcpy(stage + ray_bytes + size_t(mb[j].ray_off) * sizeof(uint32_t), it.initial_idx,
                   size_t(it.n_rays) * sizeof(uint32_t));
   });
+  WaitUnlessDone wait{s};
   HIP_TRY(r.scratch_rays.upload(reinterpret_cast<const float *>(stage), size_t(ray_total) * 6, s));
   if (with_idx)
     HIP_TRY(r.scratch_idx.upload(reinterpret_cast<const uint32_t *>(stage + ray_bytes),
@@ -889,20 +904,18 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
     rng.dim_bound = settings.max_sample_size;
     rng.initial_dim_bound = settings.max_sample_size < 64 ? settings.max_sample_size : 64;
   }
-  // (the stream is synchronised before the staging buffer is used again)
   const size_t sample_floats = size_t(n_img) * total * 3;
   HandOver hand_over{
       hand_over_paths(r, total, true, settings.max_blocks_per_launch_gpu)};
-  BatchReduction red;
-  for (uint32_t j = 0; j < m; ++j)
-    red.add(mb[j].wd, desc[j].pixel_off);
   if (r.mega_split && !r.profiling && hand_over.max_paths >= kRaysWavefrontMin &&
       (n_steps == 0 || n_steps >= 3) && sample_floats * sizeof(float) <= kRaysWavefrontBytes &&
       total >= red.alone.size() * n_img * kRaysPerReduction) {
     rc = rays_wavefront(r, items, act, desc, red, settings, rng, with_idx != 0, n_steps, total,
                         ray_total, t0, seconds, &hand_over);
-    if (!hand_over.no_memory)
+    if (!hand_over.no_memory) {
+      wait.done = rc == PT_OK;
       return rc;
+    }
   }
   HIP_TRY(r.mb_items.upload(mb.data(), m, s));
   HIP_TRY(r.mb_blocks.upload(block_begin.data(), m + 1, s));
@@ -970,6 +983,7 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
   r.stats.rays = rays_traced;
   r.stats.samples = ray_total * spp;
   r.stats.mega_launches = 1;
+  wait.done = true;
   if (seconds)
     *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return PT_OK;

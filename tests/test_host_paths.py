@@ -233,3 +233,21 @@ def test_large_values_are_given_back(fake, call, freed):
     call(r, scene)
     assert fake.fake_live() == before
     assert (values > 512 << 20) == freed and (before < 900 << 20)
+
+
+# errors after the rays' upload was queued: no Sobol table (there are no direction
+# numbers), no room for the mega-kernel's outputs, launches that fail
+@pytest.mark.parametrize("what", ["sobol", "memory", "wf_shade", "wf_reduce_batch", "mega_batch"])
+def test_failed_ray_batch_leaves_no_copies(fake, what):
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(20)
+    r.set_megakernel_split(what not in ("memory", "mega_batch"))
+    s = _settings(rng="Sobel" if what == "sobol" else "Uniform")
+    items = [(scene, _rays(4096), None)]
+    r.render_rays_batch(items, 8, 0, _settings())  # scene and staging are there
+    fake.fake_fail(what.encode())
+    if what == "memory":
+        fake.fake_limit(fake.fake_live() + 50000)
+    with pytest.raises(L.PathError):
+        r.render_rays_batch(items, 128, 8, s)
+    assert fake.fake_in_flight() == 0
