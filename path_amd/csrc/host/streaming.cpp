@@ -7,6 +7,7 @@
 #include "../gpu/wavefront.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <string>
 #include <system_error>
@@ -196,15 +197,30 @@ static hipError_t enqueue_iteration(pt_renderer &r, gpu::WfParams &p, int pipe, 
 
 // Wait until the pipeline has reported iteration `iteration` (numbered from
 // 1): its traversal has started. The stream is asked now and then, so that a
-// failed launch ends the wait.
+// failed launch ends the wait. The cores may be wanted (a program's scene
+// generation): after the first moments the thread yields, and where an iteration
+// takes long it sleeps, since the traversal that reports then runs on for longer
+// than a sleep. (From 0.1 ms on, a batch of 1.15 M ray samples and three steps took
+// 1,690 us, and 1,600 from 0.25 ms on, as without sleeps. Cores busy during 64
+// generated scenes at 128 samples: 3.1 without, 1.1 with.)
 static hipError_t wait_report(const volatile gpu::WfReport *rep, uint32_t iteration,
                               hipStream_t s) {
   auto there = [&] {
     return int32_t(__atomic_load_n(&rep->iteration, __ATOMIC_ACQUIRE) - iteration) >= 0;
   };
-  for (uint32_t spin = 1; !there(); ++spin) {
-    __builtin_ia32_pause();
-    if (spin % 8192 != 0)
+  using clock = std::chrono::steady_clock;
+  const clock::time_point sleep_from = clock::now() + std::chrono::microseconds(250);
+  bool sleeping = false;
+  for (uint32_t turn = 1; !there(); ++turn) {
+    if (sleeping) {
+      std::this_thread::sleep_for(std::chrono::microseconds(50));
+    } else if (turn % 64 != 0) {
+      __builtin_ia32_pause();
+    } else {
+      std::this_thread::yield();
+      sleeping = clock::now() >= sleep_from;
+    }
+    if (turn % (sleeping ? 16 : 8192) != 0)
       continue;
     const hipError_t e = hipStreamQuery(s);
     if (e == hipErrorNotReady)

@@ -251,3 +251,18 @@ def test_failed_ray_batch_leaves_no_copies(fake, what):
     with pytest.raises(L.PathError):
         r.render_rays_batch(items, 128, 8, s)
     assert fake.fake_in_flight() == 0
+
+
+def test_waiting_for_iterations_sleeps(fake):
+    """Three pipelines of which each waits 0.3 s for its iteration."""
+    import time
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(20)
+    s = _settings(kernel_approach="Streaming")
+    r.render(scene, FTW, 256, 256, 16, s)
+    fake.fake_report_delay(300)
+    wall, cpu = time.perf_counter(), time.process_time()
+    r.render(scene, FTW, 256, 256, 16, s)
+    assert r.last_stats().pipelines == 3
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall > 0.3 and cpu < wall  # spinning: three times the wall time
