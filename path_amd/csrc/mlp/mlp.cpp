@@ -411,13 +411,14 @@ int pt_mlp_train(pt_mlp *m, uint32_t steps, uint32_t batch, float lr, uint64_t s
     return set_error(PT_ERR_INVALID, "no training set (pt_mlp_set_dataset)");
   HIP_TRY(hipSetDevice(m->device));
   const uint32_t rp = mlp_pad_rows(batch);
-  int rc = m->ensure_training(rp, steps);
+  int rc = m->ensure_training(rp, losses ? steps : 1);
   if (rc != PT_OK)
     return rc;
   auto t0 = std::chrono::steady_clock::now();
   for (uint32_t it = 0; it < steps; ++it) {
     rc = m->gradients(m->ds_feat.ptr, m->ds_targ.ptr, m->ds_rows,
-                      seed + it * 0x632be59bd9b4e019ull, batch, rp, m->step_losses.ptr + it);
+                      seed + it * 0x632be59bd9b4e019ull, batch, rp,
+                      m->step_losses.ptr + (losses ? it : 0));
     if (rc == PT_OK)
       rc = m->update(kUpdateAdam, rp, lr);
     if (rc != PT_OK)

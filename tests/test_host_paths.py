@@ -266,3 +266,16 @@ def test_waiting_for_iterations_sleeps(fake):
     assert r.last_stats().pipelines == 3
     wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
     assert wall > 0.3 and cpu < wall  # spinning: three times the wall time
+
+
+@pytest.mark.parametrize("with_losses", [False, True])
+def test_training_keeps_losses_only_when_asked(fake, with_losses):
+    from path_amd.mlp import RadianceMLP
+    m = RadianceMLP(0)
+    m.set_dataset(np.zeros((10, 9), np.float32), np.zeros((10, 3), np.float32))
+    live = []
+    for steps in (1, 50000):
+        losses = np.zeros(steps, np.float32) if with_losses else None
+        L.check(fake.pt_mlp_train(m.handle, steps, 100, 1e-3, 1, L.fptr(losses), None))
+        live.append(fake.fake_live())
+    assert live[1] - live[0] == (4 * 49999 if with_losses else 0)
