@@ -642,7 +642,9 @@ hipError_t launch_wf_trace(const WfParams &p, WfKind kind, uint32_t grid_blocks,
 // two launches and the latency of its longest ray whatever their number. Only
 // kFinishLanes lanes of a wave take a path, so that few paths still spread over
 // the chip and wait for few others' rays. The vertices are those of wf_shade,
-// so the results are the same bits.
+// so the results are the same bits. The launch follows an iteration after which
+// no sample was left to start, so every path here has been through a shade step
+// with its first hit: given first hits and G-buffers are behind it.
 constexpr uint32_t kFinishLanes = kFinishBlockPaths / 4;
 
 template <class R, int kKind>
@@ -685,10 +687,6 @@ __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
       light_ray.d = {d.x, d.y, d.z};
     }
     R rng = make_rng<R>(p.rng, location, sample, meta.z);
-    Hit<float> given = {0.f, kNoHit, 0};
-    bool is_given = false;
-    if constexpr (kKind == kWfRays)
-      is_given = given_hit(p, meta, scene, &given);
     for (;;) {
       if (steps)
         st.total = {0.f, 0.f, 0.f};
@@ -701,24 +699,17 @@ __global__ __launch_bounds__(256) void k_wf_finish(WfParams p) {
       }
       if (st.has_next) {
         ++n_ext;
-        if (is_given)
-          next_hit = given;
-        else if (has_nodes)
+        if (has_nodes)
           next_hit = trace_closest(nodes, tris, last, 3.4028235e38f, -1.0f, stack);
       }
       PathState<float> ns;
       Ray<float> nl = light_ray, nn = last;
-      VertexInfo<float> vi;
-      vi.valid = 0u;
       bool done = rendering_equation_iteration(st, rng, last, light_hit, next_hit, p.settings,
-                                               sc.view, &ns, &nl, &nn, &vi);
-      is_given = false;
+                                               sc.view, &ns, &nl, &nn);
       if (steps) {
         write_step(p, sc, location, sample, st.iters, ns.total);
         done = done || ns.iters >= p.batch.n_steps;
       }
-      if (p.gbuffer && st.iters == 0 && sample == 0 && vi.valid)
-        write_gbuffer(p, sc, location, vi);
       if (done) {
         if (!steps)
           write_sample(p, sc, location, sample, ns.total);

@@ -7,7 +7,6 @@ namespace pt {
 namespace mlp {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -26,9 +25,6 @@ __device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
 // and gradients outside have the raw features first (column d), then feature
 // d's pairs at 9 + 24 d.
 constexpr uint32_t kEncPairs = kEncoded - kFeatures; // 216
-__host__ __device__ inline uint32_t inner_column(uint32_t c) {
-  return c < kFeatures ? kEncPairs + c : c < kEncoded ? c - kFeatures : c;
-}
 __host__ __device__ inline uint32_t outer_column(uint32_t k) {
   return k < kEncPairs ? k + kFeatures : k < kEncoded ? k - kEncPairs : k;
 }

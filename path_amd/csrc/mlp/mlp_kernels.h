@@ -81,7 +81,7 @@ struct MlpTileArgs {
   float *out_part;           // [tiles][3][256]: output layer's weight gradient
   float *loss_part;          // [tiles]
 };
-// Rows per tile: 128, or 32 for batches that would leave the chip idle.
+// Rows per tile: 128, or 64 or 32 for batches that would leave the chip idle.
 uint32_t mlp_tile_rows(uint32_t rows_pad);
 hipError_t launch_mlp_tile(const MlpTileArgs &a, uint32_t rows_pad, bool train, hipStream_t s);
 
