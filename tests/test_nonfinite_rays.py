@@ -1,7 +1,10 @@
 """Rays with a NaN component or an infinite direction hit nothing: the
 traversals skip them (ray_can_hit, core/geometry.h) instead of walking the
 whole tree. The brute-force checker, which has no such rule, agrees."""
+import ctypes as C
 import itertools
+import subprocess
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -34,6 +37,26 @@ def soup(seed, n, flat):
     return np.concatenate([v[:, 0], v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]], 1).astype(np.float32)
 
 
+def test_rule(tmp_path):
+    so = tmp_path / "ray_check.so"
+    subprocess.run(["g++", "-O2", "-std=c++20", "-ffp-contract=off", "-shared", "-fPIC",
+                    str(Path(__file__).resolve().parent / "native" / "ray_check.cpp"),
+                    "-o", str(so)], check=True)
+    lib = C.CDLL(str(so))
+
+    def can_hit(rays):
+        rays = np.ascontiguousarray(rays, np.float32)
+        out = np.zeros(len(rays), np.uint8)
+        lib.rays_can_hit(rays.ctypes.data_as(C.c_void_p), len(rays),
+                         out.ctypes.data_as(C.c_void_p))
+        return out
+    assert not can_hit(nonfinite_rays()).any()
+    # finite components of every size, and infinite origins
+    sizes = [0.0, -0.0, 1e-45, -1e-40, 1.2e-38, 0.7, -5.0, 1e20, 3.4028235e38, -3.4028235e38]
+    assert can_hit(np.array(list(itertools.product(sizes, repeat=6)), np.float32)).all()
+    assert can_hit([[np.inf, 0, -np.inf, 1, 0, 0]]).all()
+
+
 @pytest.mark.parametrize("flat", [False, True])
 def test_brute_force_finds_no_hit(flat):
     from oracle import oracle as O
@@ -58,3 +81,30 @@ def test_gpu_finds_no_hit(renderer, request, which):
     _, ridx, _ = O.loopall(scene.flat()["tris"], rays)
     assert np.array_equal(idx, ridx)
     assert (idx[at] == 0xFFFFFFFF).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps", [0, 3])
+def test_ray_batch_of_the_wavefront(renderer, cornell_sphere, steps):
+    """The wavefront's traversal writes such a ray's miss itself: a batch large
+    enough for it equals the mega-kernel's render of the same rays."""
+    from path_amd.renderer import Settings
+    from tests.helpers import random_rays
+    scene, _ = cornell_sphere
+    rays = random_rays(3000, -1.2, 2.2, seed=5)
+    bad = nonfinite_rays()
+    rays[np.random.default_rng(1).choice(len(rays), len(bad), replace=False)] = bad
+    s = Settings()
+    s.kernel_approach = "MegaKernel"
+    s.term_prob, s.n_iters = "NIters", 3
+    spp = 96
+    (got,) = renderer.render_rays_batch([(scene, rays, None)], spp, steps, s)
+    assert renderer.last_stats().mega_launches == 0
+    traced = renderer.last_stats().rays
+    out = dict(output="OutputPerStep", n_steps=steps) if steps else {}
+    ref, _ = renderer.render(scene, None, 0, 0, spp, s, rays=rays, **out)
+    assert renderer.last_stats().mega_launches > 0 and renderer.last_stats().rays == traced
+    got = np.asarray(got).reshape(max(steps, 1), len(rays), 3)
+    ref = ref.reshape(got.shape)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    assert ref.sum() > 0
