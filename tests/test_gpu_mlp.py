@@ -100,6 +100,26 @@ def test_gradient_over_tile_sizes(net, n):
         assert np.linalg.norm(a - b) <= (3e-2 if n < 32 else 1e-2) * np.linalg.norm(b)
 
 
+def test_gradient_sums_of_a_large_batch(net):
+    """262,144 rows against the FP64 mean of 128 gradients of 2,048 of them: with
+    powers of two the roundings to BF16 are the same, so only the sums over the rows
+    differ. Each weight's sum is a chain of at most rows / splits / 16 products of
+    16 rows, splits / 4 partials and 4 wave sums (42 splits); each addition rounds by
+    2^-24 of a partial sum, and here no partial sum is far above the whole."""
+    n, c = 1 << 18, 1 << 11
+    f, t = _data(n, 9)
+    g, loss = net.gradient(f, t)
+    parts = [net.gradient(f[i:i + c], t[i:i + c]) for i in range(0, n, c)]
+    ref = np.mean([p[0].astype(np.float64) for p in parts], 0)
+    bound = (n / 42 / 16 + 42 / 4 + 4) * 2.0 ** -24
+    from oracle import mlp_ref as M
+    offs = np.cumsum([0] + [o * i for o, i in M.SHAPES])
+    for l in range(len(M.SHAPES)):
+        a, b = g[offs[l]:offs[l + 1]], ref[offs[l]:offs[l + 1]]
+        assert np.linalg.norm(a - b) <= bound * np.linalg.norm(b)
+    assert abs(loss - np.mean([p[1] for p in parts])) <= bound * loss
+
+
 def test_train_draws_rows_and_steps_like_train_step(net):
     """Training on the resident set equals host batches of the rows it draws
     (SplitMix64 of the row's number), step by step."""
