@@ -384,7 +384,9 @@ int pt_render_rays_batch(pt_renderer *r, const pt_ray_batch_item *items, uint32_
  * trace_blocks_per_cu: traversal grid per pipeline = CUs x this x 256
  * threads (default 3 for a render, 6 for a batch; 0 restores the
  * defaults); iters_per_sync: iterations enqueued between host
- * checks; use_graphs: replay those iterations as one captured hipGraph. */
+ * checks; use_graphs: replay those iterations as one captured hipGraph.
+ * MegaKernel work that runs on the wavefront's kernels (pt_kernel_approach) takes
+ * the defaults of these and of the pipelines. */
 int pt_set_launch_params(pt_renderer *r, uint32_t trace_blocks_per_cu,
                          uint32_t iters_per_sync, int use_graphs);
 /* Tree builder of pt_render_batch (no reference counterpart: the reference

@@ -905,6 +905,7 @@ int render_rays_batch(pt_renderer &r, const pt_ray_batch_item *items, uint32_t n
     rng.initial_dim_bound = settings.max_sample_size < 64 ? settings.max_sample_size : 64;
   }
   const size_t sample_floats = size_t(n_img) * total * 3;
+  HandOver::Defaults defaults(r);
   HandOver hand_over{
       hand_over_paths(r, total, true, settings.max_blocks_per_launch_gpu)};
   if (r.mega_split && !r.profiling && hand_over.max_paths >= kRaysWavefrontMin &&

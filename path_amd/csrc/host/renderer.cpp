@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <atomic>
+#include <optional>
 #include <vector>
 
 using namespace pt;
@@ -393,6 +394,9 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   const float *final_rgb = nullptr;
   bool wavefront = settings.kernel_approach == PT_STREAMING;
   const uint64_t samples = uint64_t(n_pixels) * samples_per;
+  std::optional<HandOver::Defaults> defaults;
+  if (!wavefront)
+    defaults.emplace(*this);
   const uint64_t paths =
       hand_over_paths(*this, samples, false, settings.max_blocks_per_launch_gpu);
   const bool may_hand_over =

@@ -341,6 +341,28 @@ struct HandOver {
   // Gives back what the wavefront holds (but the last Streaming render's
   // samples), so that the mega-kernel finds the room it would have had.
   int does_not_fit(pt_renderer &r);
+  // Sets the wavefront's launch parameters to their defaults for a scope:
+  // pt_set_launch_params and pt_set_pipelines (and the autotuner) choose them for
+  // the Streaming integrator. (333 x 217 at 24 samples of 20,516 triangles, 2,260 us
+  // with the defaults and 3,700 on the mega-kernel: 3,950 with 16 blocks per CU,
+  // 2,940 with 64 iterations per check.)
+  struct Defaults {
+    pt_renderer &r;
+    const uint32_t blocks = r.trace_blocks_per_cu, iters = r.iters_per_sync, pipes = r.n_pipes;
+    const bool graphs = r.use_graphs;
+    explicit Defaults(pt_renderer &renderer) : r(renderer) {
+      r.trace_blocks_per_cu = 0;
+      r.iters_per_sync = 1;
+      r.n_pipes = 0;
+      r.use_graphs = false;
+    }
+    ~Defaults() {
+      r.trace_blocks_per_cu = blocks;
+      r.iters_per_sync = iters;
+      r.n_pipes = pipes;
+      r.use_graphs = graphs;
+    }
+  };
   // After a render: per-sample values above kKept are given back. (Allocating
   // and freeing 0.5 to 0.8 GB takes 0.34 ms, 2 to 4 GB 0.65 ms, where the paths
   // of so many values take more than 20 ms.)

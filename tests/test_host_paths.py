@@ -279,3 +279,25 @@ def test_training_keeps_losses_only_when_asked(fake, with_losses):
         L.check(fake.pt_mlp_train(m.handle, steps, 100, 1e-3, 1, L.fptr(losses), None))
         live.append(fake.fake_live())
     assert live[1] - live[0] == (4 * 49999 if with_losses else 0)
+
+
+# the Streaming integrator's parameters, for which hand-overs were not measured
+@pytest.mark.parametrize("params,pipes", [((16, 1, False), 0), ((0, 64, False), 0),
+                                          ((0, 1, True), 0), ((0, 1, False), 1)])
+def test_hand_over_takes_default_launch_parameters(fake, params, pipes):
+    from path_amd.datagen import set_launch_params, set_pipelines
+    from path_amd.renderer import Renderer
+    r, scene = Renderer(0), _scene(1100)
+    set_launch_params(r, *params)
+    set_pipelines(r, pipes)
+    for call, blocks in ((lambda: r.render(scene, FTW, 256, 256, 24, _settings()), 2048),
+                         (lambda: r.render_rays_batch([(scene, _rays(4096), None)], 256, 0,
+                                                      _settings()), 1536)):
+        fake.fake_reset()
+        call()
+        assert r.last_stats().pipelines == fake.fake_launches(b"wf_shade") == 3
+        assert fake.fake_blocks() == blocks
+    set_launch_params(r, 5, 3, False)
+    fake.fake_reset()
+    r.render(scene, FTW, 64, 64, 16, _settings(kernel_approach="Streaming"))
+    assert fake.fake_blocks() == 5 * 256 and fake.fake_launches(b"wf_shade") == 3
