@@ -217,7 +217,7 @@ template <uint32_t kI> constexpr size_t tile_lds(bool train) {
 // to the gradient. The MFMAs of every output element run in the K order of
 // k_gemm's and round the same way, so the forward results equal the
 // layer-by-layer GEMMs' bit for bit (GPU test).
-// Inference is bound by the matrix cores: 2^20 queries 0.61 ms, 1.35 PFLOP/s
+// Inference is bound by the matrix cores: 2^20 queries 0.60 ms, 1.34 PFLOP/s
 // (0.94 ms with row-major weights and two-byte stores of the encoding); a
 // large bf16 library product reaches 1.23 on the same card. Training at
 // 65,536 rows: 130 us for 75 us of matrix work and 0.4 GB written (one GEMM
