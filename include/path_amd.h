@@ -113,15 +113,15 @@ typedef struct pt_work_division_settings {
 
 /* The integrators give the same image bit for bit. PT_MEGA_KERNEL images of
  * many samples of a mesh (1.6 M of 1,024 triangles and depth 3 or more, 4.2 M of
- * 4,096 triangles with roulette, up to 2^26 samples), a few of whose paths show
- * that most go on for some vertices, run on the Streaming integrator's kernels, which are faster there, and so do ray batches
- * (pt_render_rays_batch) of 262,144 samples without steps or with three and
- * more, unless profiling is on, pt_set_megakernel_split is off, or
- * max_blocks_per_launch_gpu is too small for that (below 1,366 blocks, or below
- * the traversal's grid; above, none of its launches that trace or shade has
- * more blocks either). Those take device memory for the paths and their
- * values; where it does not fit, the mega-kernel runs. The renderer keeps about
- * a gigabyte of it. */
+ * 4,096 triangles with roulette, up to 2^26 samples) run on the Streaming
+ * integrator's kernels if a few of their paths show that most go on for some
+ * vertices, and so do ray batches (pt_render_rays_batch) of 262,144 samples
+ * without steps or with three and more: it is faster there. Not where profiling
+ * is on, pt_set_megakernel_split is off, or max_blocks_per_launch_gpu is below
+ * 1,366 blocks (images) or the traversal's grid (above, none of the launches that
+ * trace or shade has more blocks either). Device memory for the paths and their
+ * values is taken for it, of which the renderer keeps about a gigabyte; where it
+ * does not fit, the mega-kernel runs. */
 enum pt_kernel_approach { PT_MEGA_KERNEL = 0, PT_STREAMING = 1 };
 enum pt_accel_type {
   PT_ACCEL_LOOP_ALL = 0,

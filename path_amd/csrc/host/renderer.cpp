@@ -254,11 +254,11 @@ int pt_renderer::intersect(const pt_scene &scene, const float *rays, uint32_t n,
 }
 
 // Whether the wavefront renders a MegaKernel image (the same bits: same paths,
-// same sums) with a pool of `paths`. It keeps its lanes busy where
-// rays differ in length, but writes and reads each path's state between its
-// vertices and pays two launches an iteration: it wins with many triangles,
-// samples and rays per sample. Mega-kernel / wavefront, us, at depth 1, 4, 7 and
-// Constant 0.25 in a closed room:
+// same sums) with a pool of `paths`. It keeps its lanes busy where rays differ in
+// length, but writes and reads each path's state between its vertices and pays
+// two launches an iteration: it wins with many triangles, samples and rays per
+// sample. Mega-kernel / wavefront, us, at depth 1, 4, 7 and Constant 0.25 in a
+// closed room:
 //   356 triangles, 2.1 M samples: 656/798, 1,767/1,417, 2,877/1,912, 2,729/2,339
 //   1,316, 1.0 M: 427/607, 1,138/1,041, 1,775/1,445, 1,903/2,028
 //   5,156, 1.0 M: 505/655, 1,296/1,134, 2,077/1,591, 1,886/2,189
@@ -390,25 +390,26 @@ int pt_renderer::render(const pt_sample_spec &spec, const pt_output &out,
   stats = pt_render_stats{};
   stats.profiled = profiling ? 1u : 0u;
   auto t0 = std::chrono::steady_clock::now();
-  HIP_TRY(hipEventRecord(ev_start, stream));
   const float *final_rgb = nullptr;
   bool wavefront = settings.kernel_approach == PT_STREAMING;
   const uint64_t samples = uint64_t(n_pixels) * samples_per;
   std::optional<HandOver::Defaults> defaults;
   if (!wavefront)
     defaults.emplace(*this);
-  const uint64_t paths =
-      hand_over_paths(*this, samples, false, settings.max_blocks_per_launch_gpu);
-  const bool may_hand_over =
-      !wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split && !profiling &&
-      wavefront_may_be_faster(settings, samples, paths, scene_store.dev.n_tris);
-  const float line = wavefront_rays_per_sample(samples);
+  HandOver hand_over{hand_over_paths(*this, samples, false, settings.max_blocks_per_launch_gpu)};
+  bool faster = !wavefront && spec.type == PT_SAMPLE_SQUARE_IMAGE && !per_step && mega_split &&
+                !profiling &&
+                wavefront_may_be_faster(settings, samples, hand_over.max_paths,
+                                        scene_store.dev.n_tris);
+  if (faster) { // (the estimate takes 2 to 25 us)
+    const float line = wavefront_rays_per_sample(samples);
+    faster =
+        rays_per_sample(scene, settings, spec.film_to_world, x_dim, y_dim, line) >= line;
+  }
   if (out.type == PT_OUTPUT_BGRA) // (before the wavefront's buffers)
     HIP_TRY(bgra.ensure(n_pixels));
-  // (the estimate takes 2 to 25 us of host time)
-  if (may_hand_over && rays_per_sample(scene, settings, spec.film_to_world, x_dim, y_dim, line) >=
-                           line) {
-    HandOver hand_over{paths};
+  HIP_TRY(hipEventRecord(ev_start, stream));
+  if (faster) {
     uint64_t wf_rays = 0;
     rc = render_streaming(*this, spec, scene_store.dev, samples_per, settings, rng, x_dim, y_dim,
                           &final_rgb, &wf_rays, &hand_over);
